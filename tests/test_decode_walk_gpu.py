@@ -1,0 +1,67 @@
+"""GPU checks of the decode kernels' balanced walk (csrc/fa2_decode_walk.h) at
+the sizes where it can go wrong: lengths around the 16-key wave tiles and the
+64-key tiles the cuts count in, empty sequences, units cut into many pieces,
+row counts around the 16-row blocks and several blocks per unit.
+
+Every case passes the bars of test_decode_gpu.py (the reference tolerance, and
+errors against fp64 within 4x / 2x of the reference arithmetic's).  A forced
+split count runs one split per workgroup instead of the walk; the two differ
+by the order of fp32 sums (and, in 16 bits, by softmax weights rounded after
+different maxima), so they agree within the strict bar's own floor.
+"""
+
+import pytest
+import torch
+
+from decode_cases import LAYOUTS, make_decode_case
+from test_decode_gpu import check, run
+
+pytestmark = pytest.mark.gpu
+
+LENS = [0, 1, 15, 16, 17, 63, 64, 65, 300, 1100, 0]
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need an MI355X")
+    from kernels import _fa2
+    _fa2.lib()
+    yield
+
+
+def lens_of(layout):
+    return [1100] * 3 if layout == "dense" else LENS
+
+
+@pytest.mark.parametrize("heads,M", [((4, 4), 1), ((16, 4), 4), ((17, 1), 1), ((8, 2), 8),
+                                     ((33, 1), 1), ((8, 1), 8)],
+                         ids=["rows1", "rows16", "rows17", "rows32", "rows33", "rows64"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_walk_rows_and_lengths_f32(layout, D, heads, M):
+    QH, KVH = heads
+    case = make_decode_case(len(lens_of(layout)), QH, KVH, D, M, torch.float32, layout, seed=5100,
+                            causal=M > 1, ctx_lens=lens_of(layout))
+    check(case, layout, run(case, layout))
+
+
+@pytest.mark.parametrize("page", [1, 5, 16, 64])
+def test_walk_page_sizes_f32(page):
+    case = make_decode_case(6, 8, 2, 128, 2, torch.float32, "paged", seed=5200 + page,
+                            causal=True, kv_range=(1, 700))
+    check(case, "paged", run(case, "paged", shuffled=True, page=page))
+
+
+@pytest.mark.parametrize("n", [130, 5000])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_walk_one_sequence_in_many_pieces_f32(layout, n):
+    """One unit per kv head: every segment cuts it (up to 40 pieces)."""
+    case = make_decode_case(1, 8, 2, 64, 1, torch.float32, layout, seed=5300, ctx_lens=[n])
+    a = run(case, layout, decode=True)
+    check(case, layout, a)
+    b = run(case, layout, decode=True)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    c = run(case, layout, decode=True, num_splits=3)
+    for x, y in zip(a, c):  # 5000 fp32 additions of rounding 2^-24, either order
+        torch.testing.assert_close(x, y, rtol=0, atol=5000 ** 0.5 * 2.0 ** -24 * 4)

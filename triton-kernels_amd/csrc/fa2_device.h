@@ -151,6 +151,10 @@ struct KArgs {
   // lengths itself.
   int32_t inline_plan;
   int32_t auto_splits;
+  // Decode kernels, automatic splits: the balanced walk (fa2_decode_walk.h),
+  // walk_segs segments of at least walk_min tiles for each of walk_streams
+  // streams; 0 segments: unit blockIdx.x, split blockIdx.y.
+  int32_t walk_streams, walk_segs, walk_min;
 };
 
 constexpr int kMergeCountBits = 24;
@@ -1019,14 +1023,23 @@ __device__ __forceinline__ bool merge_count(const KArgs& a, int unit, int S, int
   if (threadIdx.x == 0) {
     uint64_t* c = a.merge_ctr + unit;
     const uint64_t tag = a.merge_tag;
+    // The first arrival replaces whatever the word held by (tag, 1); the
+    // others add.  (A compare-and-swap per arrival retries once for every
+    // other arrival: 63 pieces of one unit took 190 us to count.)
     uint64_t old = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     uint64_t cnt;
     for (;;) {
-      cnt = (old >> kMergeCountBits) == tag ? (old & ((uint64_t(1) << kMergeCountBits) - 1)) : 0;
-      const uint64_t nw = (tag << kMergeCountBits) | (cnt + 1);
-      if (__hip_atomic_compare_exchange_strong(c, &old, nw, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT))
+      if ((old >> kMergeCountBits) == tag) {
+        cnt = __hip_atomic_fetch_add(c, uint64_t(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
+              ((uint64_t(1) << kMergeCountBits) - 1);
         break;
+      }
+      if (__hip_atomic_compare_exchange_strong(c, &old, (tag << kMergeCountBits) | 1,
+                                               __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT)) {
+        cnt = 0;
+        break;
+      }
     }
     const bool last = static_cast<int>(cnt) + 1 == S;
     // the next launch with this tag (a graph replay) starts from zero; no

@@ -59,11 +59,6 @@
 #ifndef FA2_DECODE_FOLD
 #define FA2_DECODE_FOLD 1
 #endif
-// 1: fp32 decode units of at most kDecF32MaxRows rows run the VALU decode
-// kernel (see make_plan_packed); 0: the fp32-MFMA kernel
-#ifndef FA2_DECODE_F32_VALU
-#define FA2_DECODE_F32_VALU 1
-#endif
 // 1: ragged launches that fit the GPU at once run without the plan kernel
 // and merge their own splits (see make_plan); 0: plan and combine launches
 #ifndef FA2_INLINE_PLAN
@@ -73,17 +68,16 @@
 namespace fa2 {
 namespace {
 
-// fp32 decode (the fp32-MFMA kernel in packed-head mode): automatic splits
-// aim at this many workgroups per CU, keeping this many KV tiles per split
+// fp32 decode at head dims 16, 32 and 256 (the fp32 prefill kernel in
+// packed-head mode): automatic splits aim at this many workgroups per CU,
+// keeping this many KV tiles per split
 constexpr int64_t kF32DecodeWgsPerCu = 8;
 constexpr int64_t kF32DecodeMinTiles = 32;
-// the VALU fp32 decode kernel (two workgroups per CU): workgroups per CU and
-// KV tiles per split its automatic splits aim at.  Measured on MI355X (us per
-// call at 1 / 2 / 4 / 8 / 16 forced splits): d1 263 / 153 / 130 / 135 / 151,
-// s1 464 / 250 / 163 / 171 / 195, d2 634 / 480 / 492 / 526 / 607; these
-// constants pick 4, 4 and 2.
-constexpr int64_t kDecF32WgsPerCu = 4;
-constexpr int64_t kDecF32MinTiles = 32;
+// the fp32 decode kernel's balanced walk: KV tiles a workgroup takes at least.
+// Measured on MI355X (us per call at 2 / 4 / 8 tiles): one sequence of 4000
+// keys Hq32/Hkv8 D128 23.5 / 23.7 / 31.2, 4 of 100-900 keys 18.9 / 21.7 / 28.7,
+// 4 x 1023 dense 19.5 / 21.2 / 26.9; calls that fill the GPU do not change.
+constexpr int64_t kDecF32MinTiles = 2;
 
 // byte offset of the kXcds claim counters after the work list's item count
 // (within the 256 bytes reserved there; a cache line of their own)
@@ -138,7 +132,7 @@ struct Plan {
   int block_rows;   // rows per q-block of the launched kernel
   bool dec;         // packed fp16/bf16: the decode kernel
   bool f32;         // fp32 arithmetic: the fp32-MFMA kernel
-  bool decf32;      // packed fp32 with few rows per unit: the VALU decode kernel
+  bool decf32;      // packed fp32 at head_dim 64/128: the fp32 decode kernel
   bool conv;        // fp32 tensors with the reference's fp16 rounding: fp16 copies in the
                     // workspace, the 16-bit kernels, partials and an fp32 combine
   bool plan;        // ragged/paged: the plan kernel orders the work list
@@ -148,6 +142,8 @@ struct Plan {
   bool inline_plan; // ragged without the plan kernel (KArgs::inline_plan)
   bool bal;         // paged: the two-head kernel's balanced walk (pp_bal_locate)
   int64_t bal_slots;  // ... its part slots (4 per workgroup)
+  bool walk;          // decode: the balanced walk (fa2_decode_walk.h)
+  int64_t walk_streams, walk_segs, walk_min;
   int64_t max_wgs;  // cap on the persistent grid (0: none)
   uint32_t pool_bytes_k, pool_bytes_v;
   size_t off_work, off_count, off_ml, off_o, off_ctr, off_cq, off_ck, off_cv, total;
@@ -472,10 +468,15 @@ int finish_plan(const fa2_params* p, Plan* pl) {
   const bool parts = splits > 1 || pl->conv;
   if (!parts) pl->fold = false;
   pl->off_ctr = off;  // one merge word per one-head unit
-  if (pl->fold || pl->bal) off += static_cast<size_t>(pl->grid_x) * sizeof(uint64_t);
+  if (pl->walk)
+    off += static_cast<size_t>(pl->walk_streams * p->batch) * sizeof(uint64_t);
+  else if (pl->fold || pl->bal)
+    off += static_cast<size_t>(pl->grid_x) * sizeof(uint64_t);
   off = (off + 255) & ~size_t(255);
-  const size_t slots =
-      pl->bal ? static_cast<size_t>(pl->bal_slots) : parts ? static_cast<size_t>(splits) * pl->grid_x : 0;
+  const size_t slots = pl->walk  ? static_cast<size_t>(2 * pl->grid_x)  // two pieces per workgroup
+                       : pl->bal ? static_cast<size_t>(pl->bal_slots)
+                       : parts   ? static_cast<size_t>(splits) * pl->grid_x
+                                 : 0;
   pl->off_ml = off;
   off += slots * pl->part_rows * 2 * sizeof(float);
   off = (off + 255) & ~size_t(255);
@@ -511,11 +512,11 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   pl->dec = p->dtype != FA2_DTYPE_F32 && fast_dim(p->head_dim);
   pl->f32 = p->dtype == FA2_DTYPE_F32;  // decode's reference computes fp32 in fp32
   pl->conv = false;
-  // fp32 units of at most kDecF32MaxRows rows: the VALU decode kernel, whose
-  // units hold 4 or 8 rows
-  pl->decf32 = FA2_DECODE_F32_VALU && pl->f32 &&
-               (p->head_dim == 64 || p->head_dim == 128) && pl->rows <= kDecF32MaxRows;
-  pl->block_rows = pl->dec ? kDecRows : (pl->decf32 ? (pl->rows <= 4 ? 4 : 8) : kBM);
+  // fp32 at head_dim 64/128: the fp32 decode kernel, blocks of 16 or 32 rows
+  // (four 16-row blocks' accumulators do not fit its registers)
+  pl->decf32 = pl->f32 && (p->head_dim == 64 || p->head_dim == 128);
+  pl->block_rows =
+      pl->dec ? kDecRows : (pl->decf32 ? (pl->rows <= 16 ? 16 : 32) : kBM);
   const int64_t nqb = cdiv(pl->rows, pl->block_rows);
   pl->work_ub = nqb * p->batch;
   pl->npairs = pl->work_ub * p->kv_heads;
@@ -537,9 +538,8 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
     // 4 / 8 workgroups per CU and >= 8 tiles: d1 (128 units of 128 tiles)
     // 338 / 180 / 187 / 204 at 2 / 4 / 8 / 16 splits; d2 (512 units, up to
     // 128 tiles) 1730 / 1731 / 1148 / 1105 at 1 / 1 / 2 / 4 splits).
-    const int64_t target =
-        pl->dec ? cus : (pl->decf32 ? cus * kDecF32WgsPerCu : cus * kF32DecodeWgsPerCu);
-    const int64_t min_tiles = pl->dec ? 8 : (pl->decf32 ? kDecF32MinTiles : kF32DecodeMinTiles);
+    const int64_t target = pl->dec ? cus : cus * kF32DecodeWgsPerCu;
+    const int64_t min_tiles = pl->dec ? 8 : kF32DecodeMinTiles;
     const int64_t tiles = cdiv(kv_upper_bound(p), kBN);
     splits = 1;
     if (pl->npairs > 0 && pl->npairs < target) {
@@ -570,6 +570,29 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   pl->inline_plan = false;
   pl->bal = false;
   pl->bal_slots = 0;
+  // Automatic splits: the balanced walk.
+  if (pl->decf32 && p->num_splits == 0 && p->batch <= 64 * kWalkMaxPer) {
+    const int64_t cus = query_device ? cu_count_current_device() : 256;
+    const int64_t streams = p->kv_heads * nqb;
+    const int64_t min_tiles = kDecF32MinTiles;
+    const int64_t tiles = cdiv(kv_upper_bound(p), kBN) + 1;
+    const int64_t total = p->layout == FA2_LAYOUT_RAGGED ? tiles + p->batch : tiles * p->batch;
+    int64_t segs = std::max<int64_t>(1, cus / streams);
+    segs = std::min(segs, cdiv(total, min_tiles));
+    // (32-bit byte offsets into the part slots; see merge_pieces)
+    const int64_t part_bytes = 2 * streams * segs * pl->part_rows * pl->dim * 4;
+    if (total < (int64_t(1) << 30) && part_bytes < (int64_t(1) << 31) &&
+        streams * p->batch <= INT32_MAX) {
+      pl->walk = true;
+      pl->walk_streams = streams;
+      pl->walk_segs = segs;
+      pl->walk_min = min_tiles;
+      pl->plan = false;
+      pl->splits = 1;
+      pl->fold = false;
+      pl->grid_x = streams * segs;
+    }
+  }
   return finish_plan(p, pl);
 }
 
@@ -624,11 +647,11 @@ int launch_typed(KArgs a, const Plan& pl, hipStream_t st) {
   const dim3 grid(pl.grid_x, pl.splits);
   if constexpr (DT == FA2_DTYPE_F32 && (D == 64 || D == 128)) {
     if (pl.decf32) {
-      if (pl.block_rows == 4)
-        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 4>), grid, dim3(kDecF32Threads), 0, st,
+      if (pl.block_rows == 16)
+        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 1>), grid, dim3(kDecF32Threads), 0, st,
                            a);
       else
-        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 8>), grid, dim3(kDecF32Threads), 0, st,
+        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 2>), grid, dim3(kDecF32Threads), 0, st,
                            a);
       if (pl.splits > 1 && !pl.fold)
         hipLaunchKernelGGL((fa2_combine_kernel<DT, D, MODE>),
@@ -845,15 +868,18 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
   a.work = pl.plan ? reinterpret_cast<const int2*>(ws + pl.off_work) : nullptr;
   a.work_count = pl.plan ? reinterpret_cast<const int32_t*>(ws + pl.off_count) : nullptr;
   a.split_count = pl.dev_splits ? reinterpret_cast<int32_t*>(ws + pl.off_count) + 1 : nullptr;
-  const bool parts = pl.splits > 1 || pl.conv || pl.bal;
+  const bool parts = pl.splits > 1 || pl.conv || pl.bal || pl.walk;
   a.part_ml = parts ? reinterpret_cast<float*>(ws + pl.off_ml) : nullptr;
   a.part_o = parts ? reinterpret_cast<float*>(ws + pl.off_o) : nullptr;
   a.part_rows = pl.part_rows;
-  const bool merges = pl.fold || pl.bal;
+  const bool merges = pl.fold || pl.bal || pl.walk;
   a.merge_ctr = merges ? reinterpret_cast<uint64_t*>(ws + pl.off_ctr) : nullptr;
   a.merge_tag = merges ? next_merge_tag() : 0;
   a.inline_plan = pl.inline_plan ? 1 : 0;
   a.auto_splits = p->num_splits == 0 ? 1 : 0;
+  a.walk_streams = static_cast<int32_t>(pl.walk_streams);
+  a.walk_segs = pl.walk ? static_cast<int32_t>(pl.walk_segs) : 0;
+  a.walk_min = static_cast<int32_t>(pl.walk_min);
   a.pack_m = packed ? static_cast<int32_t>(p->q_len) : 0;
   a.dv = static_cast<int32_t>(p->head_dim);
   a.spin_cap = p->decode_spin_cap > 0 ? p->decode_spin_cap : kDecSpinCap;

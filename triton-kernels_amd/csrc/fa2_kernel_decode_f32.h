@@ -1,288 +1,408 @@
 // fa2_kernel_decode_f32.h - fp32 decode_attention / speculative_decode_attention
-// for units of few rows (Hq/Hkv * M <= kDecF32MaxRows): dot products on the
-// VALU, no MFMA.
+// on v_mfma_f32_16x16x4_f32, K and V streamed from HBM into registers.
 //
 // The references compute fp32 decode in fp32 (decode.py:84, 92-160;
-// speculative_decode.py:91-175).  A unit's rows are the query heads of one
-// kv head times the drafts (packed-head mode, KArgs::pack_m), here at most 8
-// (d1: 1, d2: 4, s1: 8), far fewer than a 32-row MFMA block.  The work per
-// key is R * D FMAs for S and as many for P.V against 8 * D bytes of K and V,
-// so these calls are HBM-bound with a VALU kernel as well, and every lane
-// carries useful rows:
-//   * workgroup = 4 waves; a lane holds CH head dims (CH * R <= 64 floats of
-//     q, as many of O) of one key slot: the NC = D / CH lanes of a slot split
-//     one K/V row, so a wave instruction reads KPW whole rows (KPW = 64 / NC);
-//   * per step each slot takes the next key of its stream: partial dots over
-//     CH dims, a butterfly over the slot's NC lanes, then an exact online
-//     softmax per row (running max, rescale, P) and O += P V on the lane's
-//     dims.  The loads of the next step are in flight during this one;
-//   * at the end the slots of a wave merge by a butterfly over the slot
-//     lanes and the 4 waves through LDS, in a fixed order (deterministic),
-//     into (m, l, O) per row: the output, or split partials that the last
-//     split merges (KArgs::merge_ctr, as the 16-bit decode kernel does).
+// speculative_decode.py:91-175).  A unit's rows are the query heads of one kv
+// head times the drafts (packed-head mode, KArgs::pack_m), in blocks of 16 NB
+// rows; a key costs 4 * D * 16 NB FLOP of matrix work against 8 * D bytes.
+// With one block the MFMAs could take 17 TB/s of K/V, so the kernel is bound by
+// HBM; with two (17 to 32 rows) they take about 8.6, close to what HBM gives.
+//   * Workgroup = 8 waves, one per CU.  Each wave walks its own 16-key tiles
+//     (tile i of the workgroup's range to wave i % 8) with its own (m, l, O), so
+//     all four matrix cores work whatever the row count and no barrier stands
+//     between a load and its use.
+//   * S^T = K Q^T: the A operand of k-step (i, e) is K[key][16 i + 4 g + e] for
+//     lane group g = lane / 16, key = lane % 16, so one 16-byte load of a K row
+//     feeds four MFMAs per row block straight from its registers.  Q^T lies in
+//     LDS in the same fragment order.
+//   * O^T = V^T P^T: k-step r takes key 4 g + r from lane group g, which is
+//     register r of the S^T accumulator, so P stays where the softmax left it.
+//     Lane i of a group loads V[key][64 h + 4 i ..+3]; element e feeds the dim
+//     block (h, e) of dims 64 h + 4 i + e, and register r of O^T block (h, e)
+//     holds dim 64 h + 16 g + 4 r + e.
+//   * K(t + 1) is issued once S(t) has read K(t), V(t + 1) once PV(t) has read
+//     V(t): two waves per SIMD keep 64 to 128 KB per CU in flight.  (A second
+//     K buffer, issued a phase earlier, gained 3 % on large two-block calls and
+//     spilled with one block at D = 128.)
+//   * The running max is raised, and O rescaled, only when a score passes it by
+//     2^8; the cross-lane maximum is skipped otherwise.
+//   * Rounding: with one block S is summed in eight chains and O in two levels
+//     (kFlush), so that the error against 64 bits stays at or below that of a
+//     tree over many lanes (2.1e-7 relative at 8192 keys).
+//   * The waves' states meet in LDS, added up by all threads in wave order; cut
+//     units merge through their partials (fa2_decode_walk.h).
+//
+// Measured on MI355X, us per call, against a dot-product kernel on the VALU
+// (up to 8 rows) and 32x32x2 MFMAs with one 32-row block per wave (above):
+// 16 sequences of 512-4096 keys, Hq16/Hkv4 D128, 8 drafts (32 rows): 682 -> 51;
+// 64 sequences of 512-8192 keys, Hq32/Hkv8 D128, decode: 459 -> 368 (6.1 TB/s),
+// 8 drafts: 1238 -> 462 (77 TFLOP/s); 16 x 8192 keys, 8 heads of D64, decode:
+// 124 -> 113, 8 drafts: 171 -> 120; one sequence of 4000 keys: 178 -> 24.
 #pragma once
 
-#include "fa2_kernel_lds.h"
+#include "fa2_decode_walk.h"
 
 namespace fa2 {
 
-constexpr int kDecF32MaxRows = 8;
-constexpr int kDecF32Waves = 4;
+constexpr int kDecF32Waves = 8;
 constexpr int kDecF32Threads = 64 * kDecF32Waves;
 
-template <int D, int R>
-struct DecF32Geo {
-  static constexpr int CH = (64 / R) < 16 ? 64 / R : 16;  // head dims per lane
-  static constexpr int NC = D / CH;                       // lanes per key slot
-  static constexpr int KPW = 64 / NC;                     // key slots per wave
-  static constexpr int NV = CH / 4;                       // float4 per lane and row
-  static_assert(NC >= 1 && NC <= 64 && KPW * NC == 64, "geometry");
-};
+__device__ __forceinline__ f32x4 mma16_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
-// R: the unit's row capacity (4 or 8); rows past the unit's own are zero
-template <int D, int MODE, int R>
-__global__ __launch_bounds__(kDecF32Threads, 2) void fa2_decode_f32_kernel(KArgs a) {
-  using G = DecF32Geo<D, R>;
-  constexpr int CH = G::CH, NC = G::NC, KPW = G::KPW, NV = G::NV;
-  constexpr int KPS = KPW * kDecF32Waves;  // keys per workgroup step
-
-  __shared__ float mrg_o[kDecF32Waves][R][D];   // per wave: merged O of its slots
-  __shared__ float mrg_ml[kDecF32Waves][R][2];  // and (m, l)
+// NB: 16-row blocks of a unit (block_rows = 16 NB)
+template <int D, int MODE, int NB>
+__global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs a) {
+  constexpr int DJ = D / 16;  // 16-dim groups of K and Q: 4 MFMA k-steps each
+  constexpr int DH = D / 64;  // 64-dim groups of V and O
+  constexpr int R = 16 * NB;
+  constexpr int kSChains = NB == 1 ? 8 : 2;
+  // O and l are summed over kFlush tiles at a time (NB = 1), which keeps the
+  // chains of rounded sums as short as a tree over more lanes would
+  constexpr bool kTwoLevel = NB == 1;
+  constexpr int kFlush = 2;
+  constexpr int kQBytes = NB * DJ * 64 * 16;       // Q fragments
+  // one wave's O, rows padded so that 16 lanes write 16 rows conflict-free
+  constexpr int kOPitch = (D + 4) * 4;
+  constexpr int kOBytes = R * kOPitch;
+  constexpr int kLds = kDecF32Waves * kOBytes;  // (Q first, then every wave's O)
+  static_assert(kLds >= kQBytes && kLds >= kMergePieceBytes<kDecF32Threads>, "LDS areas");
+  __shared__ __attribute__((aligned(16))) char lds[kLds];
+  __shared__ float mrg_ml[kDecF32Waves][R][2];
+  __shared__ DecSegment seg_sh;
   __shared__ int merge_flag;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int slot = lane / NC;  // key slot of the wave
-  const int c = lane % NC;     // dim chunk: dims [c * CH, c * CH + CH)
-
-  const Work w = decode_work<MODE>(a, blockIdx.x);
-  if (!w.valid) return;
-  const int split = blockIdx.y;
-  const int S = launch_splits(a);
-  if (split >= S) return;
-  const int rows = min(w.Lq - w.qblk * a.block_rows, R);
-  const int row0 = w.qblk * a.block_rows;
-  // keys of this split, in kBN-key tiles as the other kernels split them
-  const int ntiles = (w.Lk + kBN - 1) / kBN;
-  const int k_begin = ((ntiles * split) / S) * kBN;
-  const int k_end = min(((ntiles * (split + 1)) / S) * kBN, w.Lk);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15;
+  const int g = lane >> 4;
   const bool causal = a.mask != FA2_MASK_NONE;
+  const bool walk = a.walk_segs > 0;
+  const int stream = walk ? static_cast<int>(blockIdx.x) % a.walk_streams : 0;
+  const int seg_k = walk ? static_cast<int>(blockIdx.x) / a.walk_streams : 0;
 
-  // q chunk of every row, and each row's last visible key (bottom-right per
-  // draft position under the causal mask)
-  f32x4 q[R][NV];
-  int last[R];
-  const float* qp = static_cast<const float*>(a.q) + w.q_base + c * CH;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const bool ok = r < rows;
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-      q[r][v] = ok ? *reinterpret_cast<const f32x4*>(qp + static_cast<int64_t>(row0 + r) * a.q_ss +
-                                                     4 * v)
-                   : (f32x4){0.f, 0.f, 0.f, 0.f};
-    last[r] = causal ? min(w.Lk - 1, w.off + diag_row(a, row0 + r)) : w.Lk - 1;
+  DecPiece p;
+  DecSegment sg{};
+  int j = 0, us = 0;
+  if (walk) {
+    if (wave == 0) walk_locate<MODE>(a, seg_k, &seg_sh);
+    __syncthreads();
+    sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
+    sg.us = __builtin_amdgcn_readfirstlane(seg_sh.us);
+    sg.s0 = __builtin_amdgcn_readfirstlane(seg_sh.s0);
+    sg.s1 = __builtin_amdgcn_readfirstlane(seg_sh.s1);
+    sg.C = __builtin_amdgcn_readfirstlane(seg_sh.C);
+    j = sg.j;
+    us = sg.us;
+    if (!walk_piece<MODE>(a, sg, stream, seg_k, j, us, p)) return;
+  } else {
+    p.w = decode_work<MODE>(a, blockIdx.x);
+    if (!p.w.valid) return;
+    const int S = a.num_splits;
+    const int tiles = (p.w.Lk + kBN - 1) / kBN;
+    p.t0 = (tiles * static_cast<int>(blockIdx.y)) / S;
+    p.T = (tiles * (static_cast<int>(blockIdx.y) + 1)) / S - p.t0;
+    p.np = S;
+    p.mine = blockIdx.y;
+    p.us = p.W = 0;
+    p.unit = blockIdx.x;
   }
 
-  // element offset of key n's row (from the layout's K/V base), a clamped key
-  // when n is past the range (its scores are masked)
-  const float* kbase = static_cast<const float*>(a.k) + w.k_base + c * CH;
-  const float* vbase = static_cast<const float*>(a.v) + w.v_base + c * CH;
-  auto row_of = [&](int n, int64_t ss) -> int64_t {
-    n = min(n, max(k_end - 1, 0));
-    if constexpr (MODE == FA2_LAYOUT_PAGED) {
-      int pidx, poff;
-      if (a.page_shift >= 0) {
-        pidx = n >> a.page_shift;
-        poff = n & (a.page_size - 1);
+  for (;;) {
+    const Work& w = p.w;
+    const int row0 = w.qblk * R;
+    const int rows = min(w.Lq - row0, R);
+    const int k_begin = p.t0 * kBN;
+    const int k_end = min((p.t0 + p.T) * kBN, w.Lk);
+
+    // physical rows (in K and V) of key n, clamped to the range, and to the
+    // pool where its size is known (no read outside the allocation)
+    auto in_pool = [&](int row) { return a.kv_len > 0 ? min(max(row, 0), a.kv_len - 1) : row; };
+    auto krow_of = [&](int n) -> int {
+      n = max(min(n, k_end - 1), 0);
+      if constexpr (MODE == FA2_LAYOUT_PAGED) {
+        const int pidx = a.page_shift >= 0 ? n >> a.page_shift : n / a.page_size;
+        return in_pool(a.k_table[w.b * a.k_table_stride + pidx] * a.page_size +
+                       (n - pidx * a.page_size));
       } else {
-        pidx = n / a.page_size;
-        poff = n - pidx * a.page_size;
+        return n;
       }
-      const int page = a.k_table[w.b * a.k_table_stride + pidx];
-      return (static_cast<int64_t>(page) * a.page_size + poff) * ss;
-    } else {
-      return static_cast<int64_t>(n) * ss;
-    }
-  };
-  auto row_of_v = [&](int n) -> int64_t {
-    if constexpr (MODE == FA2_LAYOUT_PAGED) {
-      n = min(n, max(k_end - 1, 0));
-      int pidx, poff;
-      if (a.page_shift >= 0) {
-        pidx = n >> a.page_shift;
-        poff = n & (a.page_size - 1);
+    };
+    auto vrow_of = [&](int n) -> int {
+      n = max(min(n, k_end - 1), 0);
+      if constexpr (MODE == FA2_LAYOUT_PAGED) {
+        const int pidx = a.page_shift >= 0 ? n >> a.page_shift : n / a.page_size;
+        return in_pool(a.v_table[w.b * a.v_table_stride + pidx] * a.page_size +
+                       (n - pidx * a.page_size));
       } else {
-        pidx = n / a.page_size;
-        poff = n - pidx * a.page_size;
+        return n;
       }
-      const int page = a.v_table[w.b * a.v_table_stride + pidx];
-      return (static_cast<int64_t>(page) * a.page_size + poff) * a.v_ss;
-    } else {
-      return row_of(n, a.v_ss);
-    }
-  };
+    };
+    const float* kbase = static_cast<const float*>(a.k) + w.k_base + 4 * g;
+    const float* vbase = static_cast<const float*>(a.v) + w.v_base + 4 * l16;
 
-  float m[R], l[R];
-  f32x4 o[R][NV];
+    f32x4 kx[DJ], vx[4][DH];
+    auto load_k = [&](int row) {
+      const f32x4* kp = reinterpret_cast<const f32x4*>(kbase + static_cast<int64_t>(row) * a.k_ss);
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    m[r] = -INFINITY;
-    l[r] = 0.f;
+      for (int i = 0; i < DJ; ++i) kx[i] = __builtin_nontemporal_load(kp + 4 * i);
+    };
+    auto load_v = [&](int row16) {  // row16: the physical row of key lane % 16
 #pragma unroll
-    for (int v = 0; v < NV; ++v) o[r][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  }
+      for (int r = 0; r < 4; ++r) {
+        const int row = __shfl(row16, 4 * g + r);
+        const f32x4* vp =
+            reinterpret_cast<const f32x4*>(vbase + static_cast<int64_t>(row) * a.v_ss);
+#pragma unroll
+        for (int h = 0; h < DH; ++h) vx[r][h] = __builtin_nontemporal_load(vp + 16 * h);
+      }
+    };
 
-  f32x4 kx[NV], vx[NV];
-  auto load = [&](int k0, f32x4 (&kd)[NV], f32x4 (&vd)[NV]) {
-    const int n = k0 + wave * KPW + slot;
-    const float* kp = kbase + row_of(n, a.k_ss);
-    const float* vp = vbase + row_of_v(n);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      kd[v] = *reinterpret_cast<const f32x4*>(kp + 4 * v);
-      vd[v] = *reinterpret_cast<const f32x4*>(vp + 4 * v);
+    // first tile's loads, then Q into LDS in fragment order
+    int n0 = k_begin + wave * 16;  // this wave's tile
+    constexpr int kStep = 16 * kDecF32Waves;
+    int krow = 0, vrow = 0;
+    if (n0 < k_end) {
+      krow = krow_of(n0 + l16);
+      vrow = vrow_of(n0 + l16);
+      load_k(krow);
+      load_v(vrow);
+      krow = krow_of(n0 + kStep + l16);
+      vrow = vrow_of(n0 + kStep + l16);
     }
-  };
-  if (k_begin < k_end) load(k_begin, kx, vx);
-  for (int k0 = k_begin; k0 < k_end; k0 += KPS) {
-    f32x4 kn[NV], vn[NV];
-    if (k0 + KPS < k_end) load(k0 + KPS, kn, vn);
-    const int n = k0 + wave * KPW + slot;
-    float s[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      float acc = 0.f;
-#pragma unroll
-      for (int v = 0; v < NV; ++v)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_fmaf(q[r][v][j], kx[v][j], acc);
-      s[r] = acc;
-    }
-    // the full dot products: a butterfly over the slot's NC lanes
-#pragma unroll
-    for (int off = 1; off < NC; off <<= 1)
-#pragma unroll
-      for (int r = 0; r < R; ++r) s[r] += __shfl_xor(s[r], off);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const float x = (n < k_end && n <= last[r]) ? s[r] * a.scale_log2 : -INFINITY;
-      const float mn = fmaxf(m[r], x);
-      const float mu = (mn == -INFINITY) ? 0.f : mn;
-      const float alpha = fast_exp2(m[r] - mu);
-      const float p = fast_exp2(x - mu);
-      l[r] = l[r] * alpha + p;
-#pragma unroll
-      for (int v = 0; v < NV; ++v) o[r][v] = o[r][v] * alpha + p * vx[v];
-      m[r] = mn;
-    }
-    if (k0 + KPS < k_end) {
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        kx[v] = kn[v];
-        vx[v] = vn[v];
+    {
+      const float* qp = static_cast<const float*>(a.q) + w.q_base;
+      for (int f = tid; f < NB * DJ * 64; f += kDecF32Threads) {
+        const int fl = f & 63, fj = (f >> 6) % DJ, fn = (f >> 6) / DJ;
+        const int row = fn * 16 + (fl & 15);
+        const f32x4 x = row < rows ? *reinterpret_cast<const f32x4*>(
+                                         qp + static_cast<int64_t>(row0 + row) * a.q_ss + 16 * fj +
+                                         4 * (fl >> 4))
+                                   : (f32x4){0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<f32x4*>(lds + f * 16) = x;
       }
     }
-  }
+    int last[NB];  // last visible key of this lane's row
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+      last[nb] = causal ? min(k_end - 1, w.off + diag_row(a, row0 + nb * 16 + l16)) : k_end - 1;
+    // no key of a tile below this one is hidden from any row
+    const int full = causal ? min(k_end, w.off + 1) : k_end;
 
-  // merge two (m, l, O) states: this lane's and another's
-  auto merge = [&](int r, float m2, float l2, const f32x4 (&o2)[NV]) {
-    const float mn = fmaxf(m[r], m2);
-    const float mu = (mn == -INFINITY) ? 0.f : mn;
-    const float a1 = fast_exp2(m[r] - mu), a2 = fast_exp2(m2 - mu);
-    l[r] = l[r] * a1 + l2 * a2;
+    float m[NB], l[NB];
+    f32x4 o[NB][DH][4];
+    f32x4 o2[DH][4];  // kTwoLevel: the flushed sums
+    float l2 = 0.f;
+    int left = kFlush;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) o[r][v] = o[r][v] * a1 + o2[v] * a2;
-    m[r] = mn;
-  };
-  // the wave's slots, by a butterfly over the slot bits of the lane
+    for (int h = 0; h < DH; ++h)
 #pragma unroll
-  for (int off = NC; off < 64; off <<= 1) {
+      for (int e = 0; e < 4; ++e) o2[h][e] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      f32x4 o2[NV];
+    for (int nb = 0; nb < NB; ++nb) {
+      m[nb] = -INFINITY;
+      l[nb] = 0.f;
 #pragma unroll
-      for (int v = 0; v < NV; ++v)
+      for (int h = 0; h < DH; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o2[v][j] = __shfl_xor(o[r][v][j], off);
-      const float m2 = __shfl_xor(m[r], off), l2 = __shfl_xor(l[r], off);
-      merge(r, m2, l2, o2);
+        for (int e = 0; e < 4; ++e) o[nb][h][e] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
-  }
-  // the waves, through LDS, in wave order
-  if (slot == 0) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-#pragma unroll
-      for (int v = 0; v < NV; ++v)
-        *reinterpret_cast<f32x4*>(&mrg_o[wave][r][c * CH + 4 * v]) = o[r][v];
-      if (c == 0) {
-        mrg_ml[wave][r][0] = m[r];
-        mrg_ml[wave][r][1] = l[r];
-      }
-    }
-  }
-  __syncthreads();
-  const bool writer = wave == 0 && slot == 0;
-  if (writer) {
-#pragma unroll
-    for (int ww = 1; ww < kDecF32Waves; ++ww)
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        f32x4 o2[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-          o2[v] = *reinterpret_cast<const f32x4*>(&mrg_o[ww][r][c * CH + 4 * v]);
-        merge(r, mrg_ml[ww][r][0], mrg_ml[ww][r][1], o2);
-      }
-  }
+    __syncthreads();
 
-  if (S == 1) {
-    if (!writer) return;
-    float* op = static_cast<float*>(a.o) + w.o_base + c * CH;
+    for (; n0 < k_end; n0 += kStep) {
+      const bool more = n0 + kStep < k_end;
+      // (several chains per block: shorter sums, less rounding)
+      f32x4 s[NB], sc[NB][kSChains];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (r >= rows) continue;
-      const float inv = 1.f / l[r];  // 0/0 -> NaN for a row with no key, as the reference
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int v = 0; v < NV; ++v)
-        *reinterpret_cast<f32x4*>(op + static_cast<int64_t>(row0 + r) * a.o_ss + 4 * v) =
-            o[r][v] * inv;
-    }
-    return;
-  }
-  // split partials (m, l, unnormalised O) of the unit's rows
-  if (writer) {
-    const int64_t slot_id = static_cast<int64_t>(split) * a.part_slots + blockIdx.x;
+        for (int c = 0; c < kSChains; ++c) sc[nb][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (r >= rows || r >= a.part_rows) continue;
-      float* ml = a.part_ml + (slot_id * a.part_rows + r) * 2;
-      float* po = a.part_o + (slot_id * a.part_rows + r) * D + c * CH;
-      if (a.merge_ctr) {
-        if (c == 0) {
-          st_dev2(ml, m[r], l[r]);
+      for (int i = 0; i < DJ; ++i) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const f32x4 q = *reinterpret_cast<const f32x4*>(lds + ((nb * DJ + i) * 64 + lane) * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sc[nb][(4 * i + e) % kSChains] =
+                mma16_f32(kx[i][e], q[e], sc[nb][(4 * i + e) % kSChains]);
         }
+      }
 #pragma unroll
-        for (int v = 0; v < NV; ++v) st_dev4(po + 4 * v, o[r][v]);
-      } else {
-        if (c == 0) {
-          ml[0] = m[r];
-          ml[1] = l[r];
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int c = kSChains / 2; c > 0; c /= 2)
+#pragma unroll
+          for (int x = 0; x < c; ++x) sc[nb][x] += sc[nb][x + c];
+        s[nb] = sc[nb][0];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {
+        load_k(krow);
+        krow = krow_of(n0 + 2 * kStep + l16);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      float mx[NB];
+      bool need = false;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if (n0 + 16 > full) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[nb][r] = n0 + 4 * g + r <= last[nb] ? s[nb][r] : -INFINITY;
         }
+        mx[nb] = fmaxf(fmaxf(s[nb][0], s[nb][1]), fmaxf(s[nb][2], s[nb][3])) * a.scale_log2;
+        need |= mx[nb] > m[nb] + kRescaleThreshold;
+      }
+      if (__any(need)) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) *reinterpret_cast<f32x4*>(po + 4 * v) = o[r][v];
+        for (int nb = 0; nb < NB; ++nb) {
+          float x = mx[nb];
+          x = fmaxf(x, __shfl_xor(x, 16));
+          x = fmaxf(x, __shfl_xor(x, 32));
+          const float mn = fmaxf(m[nb], x);
+          const float alpha = fast_exp2(m[nb] - (mn == -INFINITY ? 0.f : mn));
+          m[nb] = mn;
+          l[nb] *= alpha;
+#pragma unroll
+          for (int h = 0; h < DH; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              o[nb][h][e] *= alpha;
+              if (kTwoLevel) o2[h][e] *= alpha;
+            }
+          if (kTwoLevel) l2 *= alpha;
+        }
+      }
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const float mu = m[nb] == -INFINITY ? 0.f : m[nb];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[nb][r] = fast_exp2(__builtin_fmaf(s[nb][r], a.scale_log2, -mu));
+          l[nb] += s[nb][r];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int h = 0; h < DH; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+              o[nb][h][e] = mma16_f32(vx[r][h][e], s[nb][r], o[nb][h][e]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {
+        load_v(vrow);
+        vrow = vrow_of(n0 + 2 * kStep + l16);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (kTwoLevel && --left == 0) {
+        left = kFlush;
+        l2 += l[0];
+        l[0] = 0.f;
+#pragma unroll
+        for (int h = 0; h < DH; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            o2[h][e] += o[0][h][e];
+            o[0][h][e] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          }
       }
     }
+    if constexpr (kTwoLevel) {
+      l[0] += l2;
+#pragma unroll
+      for (int h = 0; h < DH; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[0][h][e] += o2[h][e];
+    }
+
+    // merge the waves: their (m, l), then every wave's O scaled to the common
+    // max goes through LDS and all threads add up rows, in wave order
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      l[nb] += __shfl_xor(l[nb], 16);
+      l[nb] += __shfl_xor(l[nb], 32);
+      if (g == 0) {
+        mrg_ml[wave][nb * 16 + l16][0] = m[nb];
+        mrg_ml[wave][nb * 16 + l16][1] = l[nb];
+      }
+    }
+    __syncthreads();  // (also: every wave is done with Q)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      float mg = -INFINITY;
+#pragma unroll
+      for (int x = 0; x < kDecF32Waves; ++x) mg = fmaxf(mg, mrg_ml[x][nb * 16 + l16][0]);
+      const float f = fast_exp2(m[nb] - (mg == -INFINITY ? 0.f : mg));
+      char* po = lds + wave * kOBytes + (nb * 16 + l16) * kOPitch + 16 * g * 4;
+      if (nb * 16 + l16 < rows) {
+#pragma unroll
+        for (int h = 0; h < DH; ++h)
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            *reinterpret_cast<f32x4*>(po + (64 * h + 4 * x) * 4) =
+                (f32x4){o[nb][h][0][x] * f, o[nb][h][1][x] * f, o[nb][h][2][x] * f,
+                        o[nb][h][3][x] * f};
+      }
+    }
+    __syncthreads();
+    {
+      const int64_t slot = p.np == 1 ? 0
+                           : walk    ? walk_slot(a, sg.C, p.us, stream, p.mine)
+                                     : static_cast<int64_t>(p.mine) * a.part_slots + p.unit;
+      const uint32_t pr = static_cast<uint32_t>(a.part_rows);
+      const __amdgpu_buffer_rsrc_t rm = make_rsrc_uniform(a.part_ml + slot * pr * 2, pr * 8);
+      const __amdgpu_buffer_rsrc_t ro = make_rsrc_uniform(a.part_o + slot * pr * D, pr * D * 4);
+      constexpr int kTPR = D / 4;
+      const int col = (tid % kTPR) * 4;
+      for (int r = tid / kTPR; r < rows; r += kDecF32Threads / kTPR) {
+        float mg = -INFINITY;
+#pragma unroll
+        for (int x = 0; x < kDecF32Waves; ++x) mg = fmaxf(mg, mrg_ml[x][r][0]);
+        const float mu = mg == -INFINITY ? 0.f : mg;
+        float lt = 0.f;
+        f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int x = 0; x < kDecF32Waves; ++x) {
+          lt += mrg_ml[x][r][1] * fast_exp2(mrg_ml[x][r][0] - mu);
+          acc += *reinterpret_cast<const f32x4*>(lds + x * kOBytes + r * kOPitch + col * 4);
+        }
+        if (p.np == 1) {  // 0/0 -> NaN for a row with no key, as the reference
+          *reinterpret_cast<f32x4*>(static_cast<float*>(a.o) + w.o_base +
+                                    static_cast<int64_t>(row0 + r) * a.o_ss + col) =
+              acc * (1.f / lt);
+        } else {
+          if (col == 0)
+            __builtin_amdgcn_raw_buffer_store_b64(
+                (u32x2){__builtin_bit_cast(uint32_t, mg), __builtin_bit_cast(uint32_t, lt)}, rm,
+                r * 8, 0, kCpolSc1);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), ro,
+                                                 (r * D + col) * 4, 0, kCpolSc1);
+        }
+      }
+    }
+    if (p.np > 1) {
+      merge_publish();
+      __syncthreads();
+      if (merge_count(a, p.unit, p.np, &merge_flag)) {
+        if (walk)
+          merge_pieces<FA2_DTYPE_F32, D, kDecF32Threads, R>(
+              a, [&](int s) { return walk_slot(a, sg.C, p.us, stream, s); }, p.np, rows, w.o_base,
+              row0, lds);
+        else
+          merge_rows<FA2_DTYPE_F32, D, kDecF32Threads, R>(a, p.unit, p.np, rows, w.o_base, row0);
+      }
+    }
+    if (!walk) return;
+    ++j;
+    us = p.us + p.W;
+    if (!walk_piece<MODE>(a, sg, stream, seg_k, j, us, p)) return;
+    __syncthreads();  // the merge area becomes Q again
   }
-  if (!a.merge_ctr) return;  // the combine kernel merges
-  // the split that completes the unit's count merges its partials
-  merge_publish();
-  __syncthreads();
-  if (!merge_count(a, blockIdx.x, S, &merge_flag)) return;
-  merge_rows<FA2_DTYPE_F32, D, kDecF32Threads, R>(a, blockIdx.x, S, min(a.part_rows, rows),
-                                                  w.o_base, row0);
 }
 
 }  // namespace fa2
