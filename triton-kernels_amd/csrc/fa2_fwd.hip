@@ -1113,7 +1113,8 @@ extern "C" int fa2_kv_append(const fa2_kv_append_params* p, void* stream) {
   a.num_rows = static_cast<int32_t>(p->num_rows);
   a.page_size = static_cast<int32_t>(p->page_size);
   a.table_width = static_cast<int32_t>(p->table_width);
-  const int64_t grid = (p->num_rows + kAppendRows - 1) / kAppendRows;
+  a.block_rows = std::min(std::max(kAppendPieces / a.row_chunks, 1), kAppendRows);
+  const int64_t grid = (p->num_rows + a.block_rows - 1) / a.block_rows;
   hipLaunchKernelGGL(fa2_kv_append_kernel, dim3(static_cast<uint32_t>(grid)),
                      dim3(kAppendThreads), 0, static_cast<hipStream_t>(stream), a);
   return hipGetLastError() == hipSuccess ? FA2_OK : FA2_ERR_HIP;

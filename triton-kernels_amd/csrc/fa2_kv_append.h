@@ -9,20 +9,27 @@
 // benchmarks/attention.py:351-431.
 //
 // A pure copy, bound by HBM: each row is read once and written once.
-// Workgroup = 256 threads over 64 new rows: the lanes of the first wave
-// locate one row each (binary search of indptr, then the table entry) into
-// LDS; then all 256 lanes copy 16-byte pieces of K and V, several in
-// flight per lane.  A row whose logical page lies outside the table width,
-// or whose table entry is outside [0, num_pages), is not written (a caller
-// error must not become an out-of-bounds store).  Without v_new only K is
-// written.
+// Workgroup = 256 threads over as many rows as give each thread two 16-byte
+// pieces of K and of V (4 rows of 2 KB): many short workgroups, so that small
+// calls use every CU and a workgroup's chain of lookups hides behind others'
+// copies.  indptr goes to LDS first, then the lanes of the first wave locate
+// one row each (binary search, then start and table entries), then all lanes
+// copy.  Measured on MI355X (2 KB rows, us per call at 64 / 32 / 16 / 8 / 4 rows
+// per workgroup): 10k rows 41 / 26 / 20 / 20 / 21, 64 rows 23 / 14 / 14 / 14 / 14
+// (then bound by the host), 150k rows 245 / 242 / 236 / 232 / 225 (5.35 TB/s).
+//
+// A row whose logical page lies outside the table width, or whose table entry
+// is outside [0, num_pages), is not written (a caller error must not become an
+// out-of-bounds store).  Without v_new only K is written.
 #pragma once
 
 #include "fa2_device.h"
 
 namespace fa2 {
 
-constexpr int kAppendRows = 64;
+constexpr int kAppendRows = 64;  // rows per workgroup at most
+constexpr int kAppendPieces = 512;  // 16-byte pieces of K (and of V) per workgroup
+constexpr int kAppendIndptr = 512;  // sequences whose indptr fits LDS
 constexpr int kAppendThreads = 256;
 
 struct AppendArgs {
@@ -40,16 +47,25 @@ struct AppendArgs {
   int64_t num_pages;
   int32_t batch, heads, row_chunks, head_chunks;  // 16-byte pieces per row / per head
   int32_t num_rows, page_size, table_width;
+  int32_t block_rows;  // rows per workgroup, <= kAppendRows
 };
 
 __global__ __launch_bounds__(kAppendThreads) void fa2_kv_append_kernel(AppendArgs a) {
   __shared__ int64_t src_off[kAppendRows];
   __shared__ int64_t dk_off[kAppendRows];
   __shared__ int64_t dv_off[kAppendRows];
+  __shared__ int ip_sh[kAppendIndptr + 1];
   const int tid = threadIdx.x;
-  const int r0 = blockIdx.x * kAppendRows;
+  const int r0 = blockIdx.x * a.block_rows;
+  // indptr in LDS, so that the search below is no chain of global loads
+  const bool staged = a.batch <= kAppendIndptr;
+  if (staged) {
+    for (int i = tid; i <= a.batch; i += kAppendThreads) ip_sh[i] = a.indptr[i];
+    __syncthreads();
+  }
+  const int* ip = staged ? ip_sh : a.indptr;
 
-  if (tid < kAppendRows) {
+  if (tid < a.block_rows) {
     const int t = r0 + tid;
     int64_t so = -1, dk = -1, dv = -1;
     if (t < a.num_rows) {
@@ -57,14 +73,14 @@ __global__ __launch_bounds__(kAppendThreads) void fa2_kv_append_kernel(AppendArg
       int lo = 0, hi = a.batch - 1;
       while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (a.indptr[mid] <= t) lo = mid;
+        if (ip[mid] <= t) lo = mid;
         else hi = mid - 1;
       }
       const int b = lo;
-      const int j = t - a.indptr[b];
+      const int j = t - ip[b];
       const int n = (a.start ? a.start[b] : 0) + j;
       const int lp = n / a.page_size;
-      if (j >= 0 && t < a.indptr[b + 1] && n >= 0 && lp < a.table_width) {
+      if (j >= 0 && t < ip[b + 1] && n >= 0 && lp < a.table_width) {
         const int64_t pk = a.k_table[b * a.k_table_stride + lp];
         const int64_t pv = a.v_new ? a.v_table[b * a.v_table_stride + lp] : -1;
         const int64_t off = n - static_cast<int64_t>(lp) * a.page_size;
@@ -79,11 +95,11 @@ __global__ __launch_bounds__(kAppendThreads) void fa2_kv_append_kernel(AppendArg
   }
   __syncthreads();
 
-  const int rows = min(kAppendRows, a.num_rows - r0);
+  const int rows = min(a.block_rows, a.num_rows - r0);
   const int total = rows * a.row_chunks;
   // Every byte is read once and written once: non-temporal loads and stores
   // (a1: 4.70 -> 4.86 TB/s in alternating runs on one box).
-  constexpr int kUnroll = 4;
+  constexpr int kUnroll = kAppendPieces / kAppendThreads;
   for (int base = 0; base < total; base += kAppendThreads * kUnroll) {
     u32x4 kx[kUnroll], vx[kUnroll];
     int64_t kd[kUnroll], vd[kUnroll];
