@@ -32,7 +32,11 @@ from __future__ import annotations
 import torch
 
 from . import _fa2
-from ._launch import check_dtype_and_dim, enqueue, index_tensor, prep, rows_ok, table
+from ._launch import check_dtype_and_dim, enqueue, ext, index_tensor, prep, rows_ok, table
+
+# The launch goes through the C++ extension when it is built, else through
+# ctypes; both enqueue the same libfa2.so entry point with the same parameters.
+USE_EXT = True
 
 
 def decode_attention(
@@ -76,32 +80,21 @@ def decode_attention(
         _, KV_HEADS, N, _ = k.shape
         layout = _fa2.LAYOUT_DENSE
 
-    out = torch.empty_like(q)
-    _run_decode("decode_attention", q.unsqueeze(2), k, v, out.unsqueeze(2), layout=layout,
-                causal=False, batch=B, q_heads=Q_HEADS, kv_heads=KV_HEADS, head_dim=HEAD_DIM,
-                kv_indptr=kv_indptr, k_block_table=k_block_table, v_block_table=v_block_table,
-                kv_page_size=kv_page_size, num_splits=num_splits)
-    return out
+    return _decode("decode_attention", q, k, v, layout=layout, causal=False, batch=B,
+                   q_heads=Q_HEADS, kv_heads=KV_HEADS, head_dim=HEAD_DIM, kv_indptr=kv_indptr,
+                   k_block_table=k_block_table, v_block_table=v_block_table,
+                   kv_page_size=kv_page_size, num_splits=num_splits)
 
 
-def _run_decode(name, q4, k, v, out4, *, layout, causal, batch, q_heads, kv_heads, head_dim,
-                kv_indptr, k_block_table, v_block_table, kv_page_size, num_splits=0,
-                decode_spin_cap=0, workspace=None):
-    """Shared by decode_attention and speculative_decode_attention.
-
-    ``q4`` / ``out4`` are ``[B, QH, M, D]`` views; ``out4`` must be a view
-    of the caller's output so the kernels write it in place.
-    ``decode_spin_cap`` (tests only, fa2_params.decode_spin_cap) bounds the
-    decode kernel's ring waits; 0 = the library's bound.  ``workspace``
-    (tests only) is a uint8 device buffer used instead of an allocation."""
-    check_dtype_and_dim(name, q4.dtype, head_dim)
+def _check(name, dtype, k, v, *, layout, batch, q_heads, kv_heads, head_dim, kv_indptr,
+           k_block_table, v_block_table):
+    """Checks of this build, shared by both launch paths."""
+    check_dtype_and_dim(name, dtype, head_dim)
     if q_heads % kv_heads != 0:
         raise ValueError(f"{name}: q_heads ({q_heads}) must be a multiple of kv_heads "
                          f"({kv_heads})")
     if k.shape[-1] != head_dim or v.shape[-1] != head_dim or k.shape != v.shape:
         raise ValueError(f"{name}: k and v must have equal shapes with head_dim {head_dim}")
-    M = q4.shape[2]
-    dev = q4.device
     # shapes the device grid relies on (the reference does not check them)
     if layout == _fa2.LAYOUT_DENSE and k.shape[0] != batch:
         raise ValueError(f"{name}: k/v batch {k.shape[0]} != q batch {batch}")
@@ -111,6 +104,49 @@ def _run_decode(name, q4, k, v, out4, *, layout, causal, batch, q_heads, kv_head
                                         k_block_table.shape[0] < batch or
                                         v_block_table.shape[0] < batch):
         raise ValueError(f"{name}: kv_indptr and the block tables need {batch} rows")
+
+
+def _decode(name, q, k, v, *, layout, causal, batch, q_heads, kv_heads, head_dim, kv_indptr,
+            k_block_table, v_block_table, kv_page_size, num_splits):
+    """The output of decode_attention (q ``[B,QH,D]``) or
+    speculative_decode_attention (q ``[B,QH,M,D]``) after their assertions."""
+    x = ext() if USE_EXT else None
+    if x is not None:
+        _check(name, q.dtype, k, v, layout=layout, batch=batch, q_heads=q_heads,
+               kv_heads=kv_heads, head_dim=head_dim, kv_indptr=kv_indptr,
+               k_block_table=k_block_table, v_block_table=v_block_table)
+        paged = layout == _fa2.LAYOUT_PAGED
+        out = x.decode(q, k, v, layout, causal,
+                       kv_indptr if layout != _fa2.LAYOUT_DENSE else None,
+                       k_block_table if paged else None, v_block_table if paged else None,
+                       int(kv_page_size) if paged else 0, int(num_splits))
+        if out is not None:
+            return out  # (else the path below raises the library's error)
+    out = torch.empty_like(q)
+    squeeze = q.dim() == 3
+    _run_decode(name, q.unsqueeze(2) if squeeze else q, k, v,
+                out.unsqueeze(2) if squeeze else out, layout=layout, causal=causal, batch=batch,
+                q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, kv_indptr=kv_indptr,
+                k_block_table=k_block_table, v_block_table=v_block_table,
+                kv_page_size=kv_page_size, num_splits=num_splits)
+    return out
+
+
+def _run_decode(name, q4, k, v, out4, *, layout, causal, batch, q_heads, kv_heads, head_dim,
+                kv_indptr, k_block_table, v_block_table, kv_page_size, num_splits=0,
+                decode_spin_cap=0, workspace=None):
+    """The ctypes launch of decode_attention and speculative_decode_attention.
+
+    ``q4`` / ``out4`` are ``[B, QH, M, D]`` views; ``out4`` must be a view
+    of the caller's output so the kernels write it in place.
+    ``decode_spin_cap`` (tests only, fa2_params.decode_spin_cap) bounds the
+    decode kernel's ring waits; 0 = the library's bound.  ``workspace``
+    (tests only) is a uint8 device buffer used instead of an allocation."""
+    _check(name, q4.dtype, k, v, layout=layout, batch=batch, q_heads=q_heads, kv_heads=kv_heads,
+           head_dim=head_dim, kv_indptr=kv_indptr, k_block_table=k_block_table,
+           v_block_table=v_block_table)
+    M = q4.shape[2]
+    dev = q4.device
 
     if layout == _fa2.LAYOUT_PAGED and k.ndim == 4:
         # [pages, page, KVH, D] -> [pages * page, KVH, D] (decode.py:136-149

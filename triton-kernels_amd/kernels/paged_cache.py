@@ -26,7 +26,10 @@ from __future__ import annotations
 import torch
 
 from . import _fa2
-from ._launch import DTYPES, index_tensor, table
+from ._launch import DTYPES, ext, index_tensor, table
+
+# As kernels/decode.py: the C++ extension launches when it is built.
+USE_EXT = True
 
 
 def paged_kv_append(
@@ -84,6 +87,13 @@ def paged_kv_append(
     if kn.stride(-1) != 1 or (has_v and vn.stride() != kn.stride()):
         kn = kn.contiguous()
         vn = vn.contiguous() if has_v else None
+    x = ext() if USE_EXT else None
+    if x is not None:
+        rc = x.append(kc, vc, k_block_table, v_block_table if has_v else None, kn, vn,
+                      new_indptr, int(kv_page_size), start_pos)
+        if rc != 0:
+            raise _fa2.Fa2Error(rc)
+        return
     ip = index_tensor(new_indptr, dev)
     sp = index_tensor(start_pos, dev) if start_pos is not None else None
     kt = table(k_block_table, dev)

@@ -27,7 +27,7 @@ from __future__ import annotations
 import torch
 
 from . import _fa2
-from .decode import _run_decode
+from .decode import _decode
 
 
 def speculative_decode_attention(
@@ -74,9 +74,8 @@ def speculative_decode_attention(
 
     assert M <= 16, ("Speculative decode is intended for small draft lengths (M <= 16).")
 
-    out = torch.empty_like(q)
-    _run_decode("speculative_decode_attention", q, k, v, out, layout=layout, causal=causal,
-                batch=B, q_heads=Q_HEADS, kv_heads=KV_HEADS, head_dim=HEAD_DIM,
-                kv_indptr=kv_indptr, k_block_table=k_block_table, v_block_table=v_block_table,
-                kv_page_size=kv_page_size, num_splits=num_splits)
-    return out
+    return _decode("speculative_decode_attention", q, k, v, layout=layout, causal=bool(causal),
+                   batch=B, q_heads=Q_HEADS, kv_heads=KV_HEADS, head_dim=HEAD_DIM,
+                   kv_indptr=kv_indptr, k_block_table=k_block_table,
+                   v_block_table=v_block_table, kv_page_size=kv_page_size,
+                   num_splits=num_splits)
