@@ -65,3 +65,38 @@ def test_walk_one_sequence_in_many_pieces_f32(layout, n):
     c = run(case, layout, decode=True, num_splits=3)
     for x, y in zip(a, c):  # 5000 fp32 additions of rounding 2^-24, either order
         torch.testing.assert_close(x, y, rtol=0, atol=5000 ** 0.5 * 2.0 ** -24 * 4)
+
+
+# ---- 16-bit: units of up to 16 rows on the wave-streaming kernel (17: the ring kernel) ----
+
+@pytest.mark.parametrize("heads,M", [((4, 4), 1), ((8, 2), 1), ((10, 2), 1), ((16, 4), 4),
+                                     ((17, 1), 1)],
+                         ids=["rows1", "rows4", "rows5", "rows16", "rows17"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_walk_rows_and_lengths_16bit(layout, D, heads, M):
+    QH, KVH = heads
+    dt = torch.bfloat16 if D == 128 else torch.float16
+    case = make_decode_case(len(lens_of(layout)), QH, KVH, D, M, dt, layout, seed=5400,
+                            causal=M > 1, ctx_lens=lens_of(layout))
+    check(case, layout, run(case, layout))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("page", [1, 2, 5, 8, 64])
+def test_walk_page_sizes_16bit(page, D):
+    """Pages below and above the rows of one load, a size that is no power of two,
+    and (64 streams of long segments, one-row pages) windows of the table."""
+    heads = 64 if page == 1 else 4
+    case = make_decode_case(2, heads, heads, D, 2, torch.bfloat16, "paged", seed=5500 + page,
+                            causal=True, ctx_lens=[1500, 700])
+    check(case, "paged", run(case, "paged", shuffled=True, page=page))
+
+
+@pytest.mark.parametrize("n", [130, 5000])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_walk_one_sequence_in_many_pieces_16bit(layout, n):
+    case = make_decode_case(1, 8, 2, 128, 1, torch.bfloat16, layout, seed=5600, ctx_lens=[n])
+    a = run(case, layout, decode=True)
+    check(case, layout, a)
+    assert all(torch.equal(x, y) for x, y in zip(a, run(case, layout, decode=True)))

@@ -3,7 +3,8 @@
 //
 // A call's units are (sequence, kv head, q-block).  The kv heads and
 // q-blocks form a.walk_streams streams; stream s holds the units (b, s) of
-// all sequences in order, unit b weighing max(1, ceil(Lk_b / kBN)) tiles.
+// all sequences in order, unit b weighing max(1, ceil(Lk_b / TK)) tiles of TK
+// keys (64, or the 128 of one ring slot).
 // The grid is walk_streams * walk_segs workgroups: workgroup g takes stream
 // g % walk_streams and segment k = g / walk_streams of it, tiles [k C, (k +
 // 1) C) with C = ceil(total / walk_segs), at least a.walk_min.  The kv heads
@@ -28,7 +29,7 @@ constexpr int kWalkMaxPer = 64;
 // One piece of a unit for this workgroup.
 struct DecPiece {
   Work w;
-  int t0, T;     // first KV tile (kBN keys) and tile count
+  int t0, T;     // first KV tile and tile count
   int np, mine;  // pieces of the unit, this one's index
   int us, W;     // walk: the unit's start in its stream and its weight
   int unit;      // merge word
@@ -43,8 +44,9 @@ __device__ __forceinline__ int walk_len(const KArgs& a, int b) {
   return n > 0 ? n : 0;
 }
 
+template <int TK>
 __device__ __forceinline__ int walk_weight(int Lk) {
-  const int t = (Lk + kBN - 1) / kBN;
+  const int t = (Lk + TK - 1) / TK;
   return t > 1 ? t : 1;
 }
 
@@ -88,13 +90,13 @@ struct DecSegment {
 };
 
 // By one wave: the segment of workgroup (stream, k) into *sh (LDS).
-template <int MODE>
+template <int MODE, int TK>
 __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* sh) {
   const int lane = threadIdx.x & 63;
   const int segs = a.walk_segs;
   if constexpr (MODE == FA2_LAYOUT_DENSE) {
     if (lane == 0) {
-      const int W = walk_weight(a.kv_len);
+      const int W = walk_weight<TK>(a.kv_len);
       const int total = W * a.batch;
       const int C = max((total + segs - 1) / segs, a.walk_min);
       const int s0 = min(k * C, total);
@@ -109,7 +111,7 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
   const int per = (a.batch + 63) / 64;
   const int j0 = min(a.batch, lane * per), j1 = min(a.batch, j0 + per);
   int sum = 0;
-  for (int j = j0; j < j1; ++j) sum += walk_weight(walk_len<MODE>(a, j));
+  for (int j = j0; j < j1; ++j) sum += walk_weight<TK>(walk_len<MODE>(a, j));
   int incl = sum;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -123,7 +125,7 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
   if (excl <= s0 && s0 < incl) {  // one lane, or none past the end
     int us = excl, j = j0;
     for (;; ++j) {
-      const int W = walk_weight(walk_len<MODE>(a, j));
+      const int W = walk_weight<TK>(walk_len<MODE>(a, j));
       if (s0 < us + W) break;
       us += W;
     }
@@ -143,12 +145,12 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
 
 // The piece of sequence j's unit (starting at us in its stream) that falls
 // in segment g; false past the segment's end.
-template <int MODE>
+template <int MODE, int TK>
 __device__ __forceinline__ bool walk_piece(const KArgs& a, const DecSegment& g, int stream, int k,
                                            int j, int us, DecPiece& p) {
   if (us >= g.s1 || j >= a.batch) return false;
   p.w = packed_work<MODE>(a, j, stream % a.hkv, stream / a.hkv);
-  const int tiles = (p.w.Lk + kBN - 1) / kBN;
+  const int tiles = (p.w.Lk + TK - 1) / TK;
   p.us = us;
   p.W = tiles > 1 ? tiles : 1;
   const int b = max(us, g.s0), e = min(us + p.W, g.s1);
@@ -158,6 +160,23 @@ __device__ __forceinline__ bool walk_piece(const KArgs& a, const DecSegment& g, 
   p.np = (us + p.W - 1) / g.C - kf + 1;
   p.mine = k - kf;
   p.unit = j * a.walk_streams + stream;
+  return true;
+}
+
+// Split blockIdx.y of unit blockIdx.x (no walk); false: no such unit.
+template <int MODE, int TK>
+__device__ __forceinline__ bool split_piece(const KArgs& a, DecPiece& p) {
+  p.w = decode_work<MODE>(a, blockIdx.x);
+  if (!p.w.valid) return false;
+  const int S = a.num_splits;
+  const int split = blockIdx.y;
+  const int tiles = (p.w.Lk + TK - 1) / TK;
+  p.t0 = (tiles * split) / S;
+  p.T = (tiles * (split + 1)) / S - p.t0;
+  p.np = S;
+  p.mine = split;
+  p.us = p.W = 0;
+  p.unit = blockIdx.x;
   return true;
 }
 

@@ -22,6 +22,7 @@
 #include "fa2_kernel_pp.h"
 #include "fa2_kernel_short.h"
 #include "fa2_kernel_decode.h"
+#include "fa2_kernel_decode_wave.h"
 #include "fa2_kernel_decode_f32.h"
 #include "fa2_kernel_f32.h"
 #include "fa2_kv_append.h"
@@ -78,6 +79,10 @@ constexpr int64_t kF32DecodeMinTiles = 32;
 // keys Hq32/Hkv8 D128 23.5 / 23.7 / 31.2, 4 of 100-900 keys 18.9 / 21.7 / 28.7,
 // 4 x 1023 dense 19.5 / 21.2 / 26.9; calls that fill the GPU do not change.
 constexpr int64_t kDecF32MinTiles = 2;
+// ... and the 16-bit wave kernel's (us per call at 1 / 2 / 4 / 8 tiles, host
+// included: 4 x 1023 dense D128 19.4 / 18.8 / 18.9 / 19.9, one sequence of 8000
+// 21.4 / 20.7 / 20.9 / 21.5)
+constexpr int64_t kDecMinTiles = 2;
 
 // byte offset of the kXcds claim counters after the work list's item count
 // (within the 256 bytes reserved there; a cache line of their own)
@@ -570,11 +575,16 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   pl->inline_plan = false;
   pl->bal = false;
   pl->bal_slots = 0;
-  // Automatic splits: the balanced walk.
-  if (pl->decf32 && p->num_splits == 0 && p->batch <= 64 * kWalkMaxPer) {
+  // Automatic splits: the balanced walk; 16-bit units of up to kDwRows rows
+  // then run the wave-streaming kernel.  The ring kernel keeps forced split
+  // counts, wait bounds and larger units: at 32 rows two 16-row blocks per wave
+  // were slower (64 sequences of 512-8192 keys, Hq32/Hkv8 D128, 8 drafts: 207 us
+  // ring, 212-226 waves), at 4 rows the waves are faster (207 -> 189).
+  const bool wave = pl->dec && pl->rows <= kDwRows && p->decode_spin_cap == 0;
+  if ((pl->decf32 || wave) && p->num_splits == 0 && p->batch <= 64 * kWalkMaxPer) {
     const int64_t cus = query_device ? cu_count_current_device() : 256;
     const int64_t streams = p->kv_heads * nqb;
-    const int64_t min_tiles = kDecF32MinTiles;
+    const int64_t min_tiles = pl->dec ? kDecMinTiles : kDecF32MinTiles;
     const int64_t tiles = cdiv(kv_upper_bound(p), kBN) + 1;
     const int64_t total = p->layout == FA2_LAYOUT_RAGGED ? tiles + p->batch : tiles * p->batch;
     int64_t segs = std::max<int64_t>(1, cus / streams);
@@ -591,6 +601,7 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
       pl->splits = 1;
       pl->fold = false;
       pl->grid_x = streams * segs;
+      if (wave) pl->block_rows = kDwRows;
     }
   }
   return finish_plan(p, pl);
@@ -671,6 +682,10 @@ int launch_typed(KArgs a, const Plan& pl, hipStream_t st) {
     }
   }
   if constexpr (DT != FA2_DTYPE_F32 && (D == 64 || D == 128)) {
+    if (pl.dec && pl.walk) {
+      hipLaunchKernelGGL((fa2_decode_wave_kernel<DT, D, MODE>), grid, dim3(kDwThreads), 0, st, a);
+      return hipGetLastError() == hipSuccess ? FA2_OK : FA2_ERR_HIP;
+    }
     if (pl.dec) {
       FA2_LAUNCH_BUF(fa2_decode_kernel, grid, dim3(kDecThreads));
       if (pl.splits > 1 && !pl.fold)

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
   DecSegment sg{};
   int j = 0, us = 0;
   if (walk) {
-    if (wave == 0) walk_locate<MODE>(a, seg_k, &seg_sh);
+    if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
     __syncthreads();
     sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
     sg.us = __builtin_amdgcn_readfirstlane(seg_sh.us);
@@ -96,18 +96,9 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
     sg.C = __builtin_amdgcn_readfirstlane(seg_sh.C);
     j = sg.j;
     us = sg.us;
-    if (!walk_piece<MODE>(a, sg, stream, seg_k, j, us, p)) return;
-  } else {
-    p.w = decode_work<MODE>(a, blockIdx.x);
-    if (!p.w.valid) return;
-    const int S = a.num_splits;
-    const int tiles = (p.w.Lk + kBN - 1) / kBN;
-    p.t0 = (tiles * static_cast<int>(blockIdx.y)) / S;
-    p.T = (tiles * (static_cast<int>(blockIdx.y) + 1)) / S - p.t0;
-    p.np = S;
-    p.mine = blockIdx.y;
-    p.us = p.W = 0;
-    p.unit = blockIdx.x;
+    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, us, p)) return;
+  } else if (!split_piece<MODE, kBN>(a, p)) {
+    return;
   }
 
   for (;;) {
@@ -400,7 +391,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
     if (!walk) return;
     ++j;
     us = p.us + p.W;
-    if (!walk_piece<MODE>(a, sg, stream, seg_k, j, us, p)) return;
+    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, us, p)) return;
     __syncthreads();  // the merge area becomes Q again
   }
 }
