@@ -132,9 +132,10 @@ struct KArgs {
   // bound from the total KV rows), which the forward and combine kernels
   // use instead of num_splits.  null: num_splits.
   int32_t* split_count;
-  // fp32 tensors on the 16-bit kernels (q/k/v are fp16 copies): the forward
-  // kernel writes split partials even with one split, and the combine
-  // kernel writes the fp32 output from them.
+  // fp32 tensors on the two-head kernel, ragged (q/k/v are fp16 copies): the
+  // forward kernel writes split partials even with one split, and the combine
+  // kernel writes the fp32 output from them.  (The one-head kernel and the
+  // dense two-head kernel have instantiations with fp32 output.)
   int32_t part_out;
   // Split merge inside the forward kernel (no combine launch): one 64-bit
   // word per unit (part slot), (tag << kMergeCountBits) | count of the
@@ -870,7 +871,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_kernel(KArg
   }
 
   const float l_tot = sum_xor32(l_run);
-  if (S == 1 && !a.part_out) {
+  if (S == 1) {
     if (qrow < w.Lq) {
       const float inv = 1.f / l_tot;  // 0/0 -> NaN for a row with no key, as the reference
       const int64_t base = w.o_base + static_cast<int64_t>(qrow) * a.o_ss + hi * 4;

@@ -139,7 +139,7 @@ struct Plan {
   bool f32;         // fp32 arithmetic: the fp32-MFMA kernel
   bool decf32;      // packed fp32 at head_dim 64/128: the fp32 decode kernel
   bool conv;        // fp32 tensors with the reference's fp16 rounding: fp16 copies in the
-                    // workspace, the 16-bit kernels, partials and an fp32 combine
+                    // workspace, the 16-bit kernels with fp32 output
   bool plan;        // ragged/paged: the plan kernel orders the work list
   bool dev_splits;  // ... and lowers the automatic split count (KArgs::split_count)
   bool buf;         // paged: every row of the pool has a 31-bit byte offset
@@ -259,11 +259,15 @@ int make_plan(const fa2_params* p, Plan* pl, bool query_device, bool allow_conv 
               bool allow_bal = true) {
   const int64_t nqb = cdiv(p->q_len, kBM);
   // fp32 tensors of flash_attention_v2, whose reference rounds every operand
-  // to fp16 (attention.py:547, 569, 621) and keeps fp32 partials that a
-  // second kernel merges into the output (:636-746): dense and ragged calls
-  // at head_dim 64/128 convert q, k and v to fp16 copies in the workspace
-  // and run the 16-bit kernels, which write fp32 partials even unsplit;
-  // the combine kernel writes the fp32 output.  Paged pools are not copied.
+  // to fp16 (attention.py:547, 569, 621) and computes in fp32 from there: dense
+  // and ragged calls at head_dim 64/128 convert k and v (and q for the two-head
+  // kernel, which loads it ahead of its use) to fp16 copies in the workspace and
+  // run the 16-bit kernels, which write the fp32 output (with several splits, and
+  // ragged on the two-head kernel, fp32 partials that the combine kernel
+  // merges).  Paged pools are not copied.  Measured on MI355X, us per call,
+  // against copies of q, k and v and an fp32 combine in every case: 2 x 1500
+  // rows Hq16/Hkv4 D128 causal 62 -> 45, 2 x 2048 Hq32/Hkv8 135 -> 102, 700 rows
+  // Hq32/Hkv4 36 -> 24.
   pl->conv = FA2_F32_CONV && allow_conv && p->dtype == FA2_DTYPE_F32 &&
              p->arith != FA2_ARITH_FP32 && p->layout != FA2_LAYOUT_PAGED &&
              fast_dim(p->head_dim);
@@ -452,6 +456,11 @@ int make_plan(const fa2_params* p, Plan* pl, bool query_device, bool allow_conv 
   return finish_plan(p, pl);
 }
 
+// fp32 tensors whose forward kernel writes partials even unsplit (KArgs::part_out)
+bool part_out(const fa2_params* p, const Plan& pl) {
+  return pl.conv && pl.pp && p->layout == FA2_LAYOUT_RAGGED;
+}
+
 // Buffer path and workspace layout, common to both plans.
 int finish_plan(const fa2_params* p, Plan* pl) {
   const int splits = pl->splits;
@@ -470,7 +479,7 @@ int finish_plan(const fa2_params* p, Plan* pl) {
   off = (off + 255) & ~size_t(255);
   pl->off_count = off;  // the item count, the split count, the claim counters at kClaimOffset
   if (p->layout != FA2_LAYOUT_DENSE) off += 256;
-  const bool parts = splits > 1 || pl->conv;
+  const bool parts = splits > 1 || part_out(p, *pl);
   if (!parts) pl->fold = false;
   pl->off_ctr = off;  // one merge word per one-head unit
   if (pl->walk)
@@ -495,7 +504,7 @@ int finish_plan(const fa2_params* p, Plan* pl) {
     at = off;
     if (pl->conv) off += static_cast<size_t>(rows) * heads * p->head_dim * 2;
   };
-  copy(pl->off_cq, qrows, p->q_heads);
+  copy(pl->off_cq, pl->pp ? qrows : 0, p->q_heads);
   copy(pl->off_ck, kvrows, p->kv_heads);
   copy(pl->off_cv, kvrows, p->kv_heads);
   pl->total = off;
@@ -708,7 +717,16 @@ int launch_typed(KArgs a, const Plan& pl, hipStream_t st) {
           launched = true;
         } else if (pl.pp) {
           const dim3 gpp(static_cast<uint32_t>(pp_wgs), pl.splits);
-          if constexpr (MODE != FA2_LAYOUT_DENSE) {
+          bool f32_out = false;
+          if constexpr (DT == FA2_DTYPE_F16 && MODE == FA2_LAYOUT_DENSE) {
+            if (pl.conv) {
+              hipLaunchKernelGGL((fa2_fwd_pp_kernel<DT, D, MODE, true, false, false, false, true>),
+                                 gpp, dim3(kPPThreads), 0, st, a);
+              f32_out = true;
+            }
+          }
+          if (f32_out) {
+          } else if constexpr (MODE != FA2_LAYOUT_DENSE) {
             if (a.claim)
               hipLaunchKernelGGL((fa2_fwd_pp_kernel<DT, D, MODE, true, true>), gpp,
                                  dim3(kPPThreads), 0, st, a);
@@ -727,16 +745,24 @@ int launch_typed(KArgs a, const Plan& pl, hipStream_t st) {
           launched = true;
         }
       }
+      if constexpr (DT == FA2_DTYPE_F16 && MODE != FA2_LAYOUT_PAGED && D <= 128) {
+        if (!launched && pl.conv) {
+          hipLaunchKernelGGL((fa2_fwd_lds_kernel<DT, D, MODE, true, true>), grid, dim3(kThreads), 0,
+                             st, a);
+          launched = true;
+        }
+      }
       if (!launched) FA2_LAUNCH_BUF(fa2_fwd_lds_kernel, grid, dim3(kThreads));
     }
   }
   if (generic) FA2_LAUNCH_BUF(fa2_fwd_kernel, grid, dim3(kThreads));
   const dim3 cgrid(pl.grid_x, cdiv(pl.part_rows, kCombineRows<D>));
-  if (a.part_out) {  // fp32 output of fp16 copies (Plan::conv)
-    hipLaunchKernelGGL((fa2_combine_kernel<FA2_DTYPE_F32, D, MODE>), cgrid, dim3(kThreads), 0, st,
-                       a);
-  } else if (pl.splits > 1 && !pl.fold) {
-    hipLaunchKernelGGL((fa2_combine_kernel<DT, D, MODE>), cgrid, dim3(kThreads), 0, st, a);
+  if (a.part_out || (pl.splits > 1 && !pl.fold)) {
+    if (pl.conv)  // fp32 output
+      hipLaunchKernelGGL((fa2_combine_kernel<FA2_DTYPE_F32, D, MODE>), cgrid, dim3(kThreads), 0, st,
+                         a);
+    else
+      hipLaunchKernelGGL((fa2_combine_kernel<DT, D, MODE>), cgrid, dim3(kThreads), 0, st, a);
   }
   return hipGetLastError() == hipSuccess ? FA2_OK : FA2_ERR_HIP;
 }
@@ -883,7 +909,7 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
   a.work = pl.plan ? reinterpret_cast<const int2*>(ws + pl.off_work) : nullptr;
   a.work_count = pl.plan ? reinterpret_cast<const int32_t*>(ws + pl.off_count) : nullptr;
   a.split_count = pl.dev_splits ? reinterpret_cast<int32_t*>(ws + pl.off_count) + 1 : nullptr;
-  const bool parts = pl.splits > 1 || pl.conv || pl.bal || pl.walk;
+  const bool parts = pl.splits > 1 || part_out(p, pl) || pl.bal || pl.walk;
   a.part_ml = parts ? reinterpret_cast<float*>(ws + pl.off_ml) : nullptr;
   a.part_o = parts ? reinterpret_cast<float*>(ws + pl.off_o) : nullptr;
   a.part_rows = pl.part_rows;
@@ -901,8 +927,8 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
 
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (pl.conv) {
-    // q, k, v -> contiguous fp16 copies ([B][H][L][D] dense, [T][H][D]
-    // ragged), then the 16-bit kernels with an fp32 combine
+    // k, v (and q) -> contiguous fp16 copies ([B][H][L][D] dense, [T][H][D]
+    // ragged), then the 16-bit kernels
     const bool dense = p->layout == FA2_LAYOUT_DENSE;
     const int64_t D = p->head_dim;
     uint16_t* cq = reinterpret_cast<uint16_t*>(ws + pl.off_cq);
@@ -928,6 +954,7 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
     };
     ConvArgs c;
     c.seg[0] = seg(p->q, p->q_sb, p->q_sh, p->q_ss, p->q_len, p->q_heads, cq);
+    if (!pl.pp) c.seg[0].rows = 0;  // the one-head kernel rounds Q itself
     c.seg[1] = seg(p->k, p->k_sb, p->k_sh, p->k_ss, p->kv_len, p->kv_heads, ck);
     c.seg[2] = seg(p->v, p->v_sb, p->v_sh, p->v_ss, p->kv_len, p->kv_heads, cv);
     const int64_t rows = c.seg[0].rows + c.seg[1].rows + c.seg[2].rows;
@@ -948,13 +975,15 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
         sb = 0; sh = D; ss = heads * D;
       }
     };
-    a.q = cq;
+    if (pl.pp) {
+      a.q = cq;
+      strides(p->q_len, p->q_heads, a.q_sb, a.q_sh, a.q_ss);
+    }
     a.k = ck;
     a.v = cv;
-    strides(p->q_len, p->q_heads, a.q_sb, a.q_sh, a.q_ss);
+    a.part_out = part_out(p, pl) ? 1 : 0;
     strides(p->kv_len, p->kv_heads, a.k_sb, a.k_sh, a.k_ss);
     strides(p->kv_len, p->kv_heads, a.v_sb, a.v_sh, a.v_ss);
-    a.part_out = 1;
     return launch_dim<FA2_DTYPE_F16>(pl.dim, p->layout, a, pl, st);
   }
   switch (p->dtype) {

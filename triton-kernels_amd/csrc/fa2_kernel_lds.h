@@ -487,6 +487,41 @@ __device__ __forceinline__ void store_o_staged_buf(const f32x16 (&o)[D / 32], fl
   }
 }
 
+// fp32 output (fp32 tensors on the 16-bit kernels): the wave's 32 x D tile,
+// normalised, through LDS in passes of 32 dims (OStage<64>::kBytes: rows of 128
+// bytes plus the pad), out as 16-byte pieces of whole 128-byte runs.  `out`
+// starts at the tile's first row and covers its rows < Lq; every store is
+// issued (kOStoreOpsF32<D> vmcnt contributions).
+template <int D>
+constexpr int kOStoreOpsF32 = (D / 32) * (kWaveRows * 32 * 4 / 1024);
+
+template <int D>
+__device__ __forceinline__ void store_o_staged_f32(const f32x16 (&o)[D / 32], float inv,
+                                                   char* stage, __amdgpu_buffer_rsrc_t out,
+                                                   int64_t o_ss, int lane) {
+  constexpr int kS = OStage<64>::kStride;
+  static_assert(kS == 32 * 4 + 16, "row pitch");
+  const int l32 = lane & 31, hi = lane >> 5;
+  const uint32_t rs = static_cast<uint32_t>(o_ss * 4);
+  lds_char_t* st = to_lds(stage);
+#pragma unroll
+  for (int d = 0; d < D / 32; ++d) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(lds_u32x4_t*)(st + l32 * kS + (g * 8 + hi * 4) * 4) = __builtin_bit_cast(
+          u32x4, (f32x4){o[d][g * 4 + 0] * inv, o[d][g * 4 + 1] * inv, o[d][g * 4 + 2] * inv,
+                         o[d][g * 4 + 3] * inv});
+    u32x4 v[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it)
+      v[it] = *(const lds_u32x4_t*)(st + (it * 8 + lane / 8) * kS + (lane % 8) * 16);
+#pragma unroll
+    for (int it = 0; it < 4; ++it)
+      __builtin_amdgcn_raw_buffer_store_b128(
+          v[it], out, (it * 8 + lane / 8) * rs + (d * 32 + (lane % 8) * 4) * 4, 0, kStoreNT);
+  }
+}
+
 // Wait for this wave's outstanding direct-to-LDS loads (vmcnt), then barrier.
 __device__ __forceinline__ void lds_fill_barrier() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -508,7 +543,9 @@ __device__ __forceinline__ void lds_fill_barrier() {
 #ifndef FA2_SGB
 #define FA2_SGB 7
 #endif
-template <int DT, int D, int MODE, bool BUF, bool PIPE = FA2_LDS_PIPE_DEFAULT(D)>
+// F32: fp32 tensors (Plan::conv): K and V are fp16 copies, Q is fp32 and rounded
+// to fp16 here, an unsplit unit writes the fp32 output.
+template <int DT, int D, int MODE, bool BUF, bool F32 = false, bool PIPE = FA2_LDS_PIPE_DEFAULT(D)>
 __global__ __launch_bounds__(kThreads, D > 128 ? 1 : FA2_LDS_OCCUPANCY) void fa2_fwd_lds_kernel(KArgs a) {
   static_assert(DT != FA2_DTYPE_F32, "fp32 uses the register-staged kernel");
   constexpr bool BF = Elt<DT>::kBF;
@@ -559,12 +596,13 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : FA2_LDS_OCCUPANCY) void fa2
     const int64_t base = w.q_base + static_cast<int64_t>(qrow) * a.q_ss + hi * 8;
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
-      Raw8<DT> r;
+      constexpr int QT = F32 ? FA2_DTYPE_F32 : DT;
+      Raw8<QT> r;
       if (ok)
-        load_raw8<DT>(r, a.q, base + c * 16);
+        load_raw8<QT>(r, a.q, base + c * 16);
       else
-        zero_raw8<DT>(r);
-      qf[c] = to16<DT>(r);
+        zero_raw8<QT>(r);
+      qf[c] = to16<QT>(r);
     }
   }
 
@@ -773,10 +811,19 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : FA2_LDS_OCCUPANCY) void fa2
   }
 
   const float l_tot = sum_xor32(l_run);
-  if (S == 1 && !a.part_out) {
+  if (S == 1) {
     static_assert(kWaves * OStage<D>::kBytes <= sizeof(lds), "O staging exceeds LDS");
     __syncthreads();  // the last tile's buffers may still be read by other waves
     const float inv = 1.f / l_tot;  // 0/0 -> NaN for a row with no key, as the reference
+    if constexpr (F32) {
+      const int wrow = __builtin_amdgcn_readfirstlane(wq_first);
+      const int nrows = max(0, min(w.Lq - wrow, kWaveRows));
+      const __amdgpu_buffer_rsrc_t out = make_rsrc_uniform(
+          static_cast<float*>(a.o) + w.o_base + static_cast<int64_t>(wrow) * a.o_ss,
+          static_cast<uint32_t>(nrows) * static_cast<uint32_t>(a.o_ss * 4));
+      store_o_staged_f32<D>(o, inv, lds + wave * OStage<64>::kBytes, out, a.o_ss, lane);
+      return;
+    }
     store_o_staged<DT, D>(o, inv, lds + wave * OStage<D>::kBytes, a.o, w.o_base, a.o_ss,
                           wq_first, w.Lq, lane);
   } else {

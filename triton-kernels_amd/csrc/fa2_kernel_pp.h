@@ -186,8 +186,10 @@ __device__ void pp_bal_locate(const KArgs& a, int x, int upp, int ns, int k, int
 // instantiation for the same reason.
 // BAL: the balanced walk (pp_bal_locate), paged launches without a plan
 // kernel, one split; likewise separate.
+// F32: dense fp32 tensors (Plan::conv): q, k and v are fp16 copies, an unsplit
+// unit writes the fp32 output.
 template <int DT, int D, int MODE, bool BUF, bool CLAIM = false, bool INLINE = false,
-          bool BAL = false>
+          bool BAL = false, bool F32 = false>
 __global__ __launch_bounds__(kPPThreads, 1) void fa2_fwd_pp_kernel(KArgs a) {
   static_assert(DT != FA2_DTYPE_F32, "fp32 uses the register-staged kernel");
   static_assert(!INLINE || (MODE == FA2_LAYOUT_RAGGED && !CLAIM), "inline plans: ragged, static walk");
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa2_fwd_pp_kernel(KArgs a) {
   constexpr int kTile = G::kTileBytes;
   constexpr int kSlotBytes = 2 * kPPSlots * kTile;
   constexpr int kStageDims = 64;  // output staged in passes of 64 dims
-  constexpr int kStores = kOStoreOps<D, kStageDims>;
+  constexpr int kStores = F32 ? kOStoreOpsF32<D> : kOStoreOps<D, kStageDims>;
 
   // K/V slots, then one output staging region per wave (separate, so the
   // next unit's tiles can land while this unit's rows are being stored)
@@ -668,7 +670,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa2_fwd_pp_kernel(KArgs a) {
       // prefetch count the staged output stores)
       // (a piece of the balanced walk that writes partials waits for all of
       // them, and one that merges waits for its loads, before its stores)
-      pre_next = has_next && nxt.T > 0 && S == 1 && !a.part_out;
+      pre_next = has_next && nxt.T > 0 && S == 1 && (F32 || !a.part_out);
       // Q of the next unit: this group's last S is done
       if (pre_next) load_q(nxt);
       phase_v(T - 1);
@@ -707,6 +709,13 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa2_fwd_pp_kernel(KArgs a) {
     auto store_out = [&](const f32x16 (&v)[DB], float l) {
       const float inv = 1.f / l;  // 0/0 -> NaN for a row with no key, as the reference
       const int nrows = max(0, min(w.Lq - wq_first, kWaveRows));
+      if constexpr (F32) {
+        const __amdgpu_buffer_rsrc_t out = make_rsrc_uniform(
+            static_cast<float*>(a.o) + u.o_base + static_cast<int64_t>(wq_first) * a.o_ss,
+            static_cast<uint32_t>(nrows) * static_cast<uint32_t>(a.o_ss * 4));
+        store_o_staged_f32<D>(v, inv, stage, out, a.o_ss, lane);
+        return;
+      }
       const __amdgpu_buffer_rsrc_t out = make_rsrc_uniform(
           static_cast<uint16_t*>(a.o) + u.o_base + static_cast<int64_t>(wq_first) * a.o_ss,
           static_cast<uint32_t>(nrows) * static_cast<uint32_t>(a.o_ss * 2));
@@ -787,7 +796,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa2_fwd_pp_kernel(KArgs a) {
       }
     } else if (u.hok) {
       const float l_tot = sum_xor32(l_run);
-      if (S == 1 && !a.part_out) {
+      if (S == 1 && (F32 || !a.part_out)) {
         store_out(o, l_tot);
       } else {
         // partials go to the slot the one-head-per-unit layout gives this
