@@ -100,3 +100,17 @@ def test_walk_one_sequence_in_many_pieces_16bit(layout, n):
     a = run(case, layout, decode=True)
     check(case, layout, a)
     assert all(torch.equal(x, y) for x, y in zip(a, run(case, layout, decode=True)))
+
+
+# ---- short units, which stay whole: up to 12 tiles of 64 keys in 16 bits, 6 in fp32 ----
+
+@pytest.mark.parametrize("dt,top", [(torch.bfloat16, 12 * 64), (torch.float16, 12 * 64),
+                                    (torch.float32, 6 * 64)], ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("past", [0, 1], ids=["whole", "cut"])
+def test_short_units_stay_whole(layout, dt, top, past):
+    """The longest unit at the limit and one key past it; 128 kv heads leave two
+    segments per stream, so that a workgroup walks several units."""
+    lens = [top + past] * 5 if layout == "dense" else [top + past, 0, 1, 64, 65, 300, 17, 0, 130]
+    case = make_decode_case(len(lens), 128, 128, 64, 2, dt, layout, seed=5700, ctx_lens=lens)
+    check(case, layout, run(case, layout))

@@ -15,6 +15,14 @@
 // to finish merges, in piece order (merge_count, merge_rows_at): the cut
 // points follow from the lengths alone, so results do not depend on timing.
 //
+// When no unit has more than WHOLE tiles, cutting one costs more than it saves:
+// workgroup (s, k) then takes the whole units k, k + walk_segs, ... of its stream.
+// Measured on MI355X (us per call, always cut / whole up to 6 / up to 12 tiles):
+// 16-bit, 3 x 133 keys 16.6 / 8.2 / 8.1, 4 x 517 18.3 / 18.6 / 10.0, 64 x 16-600
+// 28.6 / 28.8 / 21.6; fp32, 8 x 20-300 keys 17.9 / 15.4 / 15.3, 4 x 517 16.9 /
+// 17.3 / 22.0.  The 16-bit kernel takes 12, the fp32 kernel, whose tiles take
+// longer, 6.
+//
 // Without a walk (walk_segs == 0, a forced split count) workgroup (x, y) runs
 // split y of unit x.
 #pragma once
@@ -84,19 +92,23 @@ __device__ __forceinline__ Work packed_work(const KArgs& a, int b, int kvh, int 
 }
 
 // The first piece's place, from walk_locate: sequence, the unit's start in
-// the stream, the segment [s0, s1) and C.
+// the stream, the segment [s0, s1) and C; C == 0: whole units.
 struct DecSegment {
   int j, us, s0, s1, C;
 };
 
 // By one wave: the segment of workgroup (stream, k) into *sh (LDS).
-template <int MODE, int TK>
+template <int MODE, int TK, int WHOLE>
 __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* sh) {
   const int lane = threadIdx.x & 63;
   const int segs = a.walk_segs;
   if constexpr (MODE == FA2_LAYOUT_DENSE) {
     if (lane == 0) {
       const int W = walk_weight<TK>(a.kv_len);
+      if (W <= WHOLE) {
+        *sh = DecSegment{k, 0, 0, 0, 0};
+        return;
+      }
       const int total = W * a.batch;
       const int C = max((total + segs - 1) / segs, a.walk_min);
       const int s0 = min(k * C, total);
@@ -110,13 +122,22 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
   }
   const int per = (a.batch + 63) / 64;
   const int j0 = min(a.batch, lane * per), j1 = min(a.batch, j0 + per);
-  int sum = 0;
-  for (int j = j0; j < j1; ++j) sum += walk_weight<TK>(walk_len<MODE>(a, j));
+  int sum = 0, longest = 0;
+  for (int j = j0; j < j1; ++j) {
+    const int W = walk_weight<TK>(walk_len<MODE>(a, j));
+    sum += W;
+    longest = max(longest, W);
+  }
   int incl = sum;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     const int y = __shfl_up(incl, d);
     if (lane >= d) incl += y;
+    longest = max(longest, __shfl_xor(longest, d));
+  }
+  if (longest <= WHOLE) {
+    if (lane == 0) *sh = DecSegment{k, 0, 0, 0, 0};
+    return;
   }
   const int total = __shfl(incl, 63);
   const int C = max((total + segs - 1) / segs, a.walk_min);
@@ -144,23 +165,36 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
 }
 
 // The piece of sequence j's unit (starting at us in its stream) that falls
-// in segment g; false past the segment's end.
+// in segment g (whole units: all of it); false past the segment's end.
 template <int MODE, int TK>
 __device__ __forceinline__ bool walk_piece(const KArgs& a, const DecSegment& g, int stream, int k,
                                            int j, int us, DecPiece& p) {
-  if (us >= g.s1 || j >= a.batch) return false;
+  const bool whole = g.C == 0;
+  if (j >= a.batch || (!whole && us >= g.s1)) return false;
   p.w = packed_work<MODE>(a, j, stream % a.hkv, stream / a.hkv);
   const int tiles = (p.w.Lk + TK - 1) / TK;
   p.us = us;
   p.W = tiles > 1 ? tiles : 1;
+  p.unit = j * a.walk_streams + stream;
+  if (whole) {
+    p.t0 = 0;
+    p.T = tiles;
+    p.np = 1;
+    p.mine = 0;
+    return true;
+  }
   const int b = max(us, g.s0), e = min(us + p.W, g.s1);
   p.t0 = b - us;
   p.T = tiles > 0 ? e - b : 0;
   const int kf = us / g.C;
   p.np = (us + p.W - 1) / g.C - kf + 1;
   p.mine = k - kf;
-  p.unit = j * a.walk_streams + stream;
   return true;
+}
+
+// The sequence whose unit follows that of sequence b in segment g.
+__device__ __forceinline__ int walk_next(const KArgs& a, const DecSegment& g, int b) {
+  return b + (g.C == 0 ? a.walk_segs : 1);
 }
 
 // Split blockIdx.y of unit blockIdx.x (no walk); false: no such unit.

@@ -46,6 +46,7 @@ namespace fa2 {
 
 constexpr int kDecF32Waves = 8;
 constexpr int kDecF32Threads = 64 * kDecF32Waves;
+constexpr int kDecF32Whole = 6;  // units of up to this many 64-key tiles stay whole
 
 __device__ __forceinline__ f32x4 mma16_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
   DecSegment sg{};
   int j = 0, us = 0;
   if (walk) {
-    if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
+    if (wave == 0) walk_locate<MODE, kBN, kDecF32Whole>(a, seg_k, &seg_sh);
     __syncthreads();
     sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
     sg.us = __builtin_amdgcn_readfirstlane(seg_sh.us);
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
       }
     }
     if (!walk) return;
-    ++j;
+    j = walk_next(a, sg, j);
     us = p.us + p.W;
     if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, us, p)) return;
     __syncthreads();  // the merge area becomes Q again

@@ -29,9 +29,9 @@
 // fa2_kernel_decode.h with a plan kernel or splits: 64 sequences of 512-8192
 // keys Hq32/Hkv8 D128 208 -> 189 (6.15 TB/s; a plain read reaches 6.9), 16 x
 // 8200 keys, 8 heads of D64, 8 drafts 69 -> 58, one sequence of 8000 keys
-// 41 -> 21, 4 x 1023 dense 17.5 -> 12.5.  What is left is uneven service: equal
-// shares end 119 to 184 us into the first of these calls, by kv head (the
-// channels its rows fall on) and by XCD.
+// 41 -> 21, 4 x 1023 dense 17.5 -> 12.5.  What is left is uneven service:
+// equal shares end 119 to 184 us into the first of these calls, by kv head
+// (the channels its rows fall on) and by XCD.
 #pragma once
 
 #include "fa2_decode_walk.h"
@@ -41,6 +41,7 @@ namespace fa2 {
 
 constexpr int kDwWaves = 8;
 constexpr int kDwThreads = 64 * kDwWaves;
+constexpr int kDwWhole = 12;      // units of up to this many 64-key tiles stay whole
 constexpr int kDwTable = 512;     // block-table entries of a window (K and V each)
 constexpr int kDwRows = 16;       // rows of a unit at most
 // rows that pass through LDS at once beside the tiles in flight
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(kDwThreads, 1) void fa2_decode_wave_kernel(KArgs a)
   const int stream = static_cast<int>(blockIdx.x) % a.walk_streams;
   const int seg_k = static_cast<int>(blockIdx.x) / a.walk_streams;
 
-  if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
+  if (wave == 0) walk_locate<MODE, kBN, kDwWhole>(a, seg_k, &seg_sh);
   __syncthreads();
   DecSegment sg;
   sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(kDwThreads, 1) void fa2_decode_wave_kernel(KArgs a)
       window_at(v, c.kb);
       return true;
     }
-    return first_window(v, c.p.w.b + 1, c.p.us + c.p.W);
+    return first_window(v, walk_next(a, sg, c.p.w.b), c.p.us + c.p.W);
   };
   auto load_table = [&](const Window& v, int buf) {
     if constexpr (kPaged) {
