@@ -143,6 +143,26 @@ def test_inline_plan_equals_plan_kernel(heads, causal, splits):
     check_all(case, "ragged", causal, unpack(case, "ragged", inline, kw))
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("longest", [300, 3000], ids=["cancelled", "running"])
+def test_inline_plan_with_splits_past_the_resident_ones(longest, causal):
+    """22 sequences of short keys, 176 units and three splits by the host's
+    bound: more workgroups than fit at once.  The lengths cancel the splits, or
+    (one longer sequence) leave two of them; either way the outcome is the plan
+    and combine kernels' bit for bit."""
+    kv = [100 + 13 * i for i in range(21)] + [longest]
+    q_lens = [longest if causal and n == longest else min(n, 17 + 5 * i)
+              for i, n in enumerate(kv)]
+    kv = q_lens if causal else kv
+    case = make_case(len(kv), 8, 2, 128, "self" if causal else "cross", torch.bfloat16,
+                     "ragged", 5450 + longest + int(causal), q_lens=q_lens, kv_lens=kv)
+    print(f"inline plan past resident causal={causal} longest={longest}", flush=True)
+    inline, kw = run(case, "ragged", causal, 0)
+    planned, _ = run(case, "ragged", causal, 0, max_workgroups=1 << 20)
+    assert same(inline, planned)
+    check_all(case, "ragged", causal, unpack(case, "ragged", inline, kw))
+
+
 @pytest.mark.parametrize("layout", ["dense", "paged"])
 @pytest.mark.parametrize("causal", [False, True])
 def test_kernel_choice_by_grid_fill_keeps_bits(layout, causal):
