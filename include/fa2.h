@@ -159,9 +159,10 @@ typedef struct fa2_params {
 
   int32_t arith;      /* enum fa2_arith (fp32 tensors only)                    */
 
-  /* fa2_decode_fwd, fp16/bf16: polls after which a wait of the decode
-   * kernel's producer/consumer ring gives up (0 = the library's bound, about
-   * 5 ms).  A wait that gives up poisons its rows with NaN and counts in
+  /* fa2_decode_fwd, fp16/bf16: polls after which a wait of the
+   * producer/consumer ring kernel gives up (0 = the library's bound, about
+   * 5 ms; another value also selects that kernel, which otherwise serves
+   * forced splits and units of more than 16 rows).  A wait that gives up poisons its rows with NaN and counts in
    * fa2_decode_wait_giveups().  Only tests set it, to exercise that path from
    * the host.  No counterpart in the reference, whose decode kernels do not
    * synchronise waves. */
@@ -188,7 +189,8 @@ enum fa2_kernel {
 /* Bytes of device workspace fa2_fwd needs for `p` (0 is possible).
  * Replaces the reference's per-call torch.empty of running_sum/max/acc
  * (attention.py:852-864).  fp32 tensors with FA2_ARITH_REFERENCE at
- * head_dim 64/128 (dense, ragged) also hold fp16 copies of q, k and v there,
+ * head_dim 64/128 (dense, ragged) also hold fp16 copies of k and v, and of q where a
+ * two-head kernel serves them, there,
  * as the reference rounds every fp32 operand to fp16.  Paged calls with one
  * q-block per sequence and more two-head units than compute units hold the
  * partials of units their balanced walk cuts into pieces (4 * CUs * 128 *

@@ -34,7 +34,7 @@
 //
 // Measured on MI355X, us per call, against a dot-product kernel on the VALU
 // (up to 8 rows) and 32x32x2 MFMAs with one 32-row block per wave (above):
-// 16 sequences of 512-4096 keys, Hq16/Hkv4 D128, 8 drafts (32 rows): 682 -> 51;
+// 16 sequences of 512-4096 keys, Hq16/Hkv4 D128, 8 drafts (32 rows): 806 -> 49;
 // 64 sequences of 512-8192 keys, Hq32/Hkv8 D128, decode: 459 -> 368 (6.1 TB/s),
 // 8 drafts: 1238 -> 462 (77 TFLOP/s); 16 x 8192 keys, 8 heads of D64, decode:
 // 124 -> 113, 8 drafts: 171 -> 120; one sequence of 4000 keys: 178 -> 24.

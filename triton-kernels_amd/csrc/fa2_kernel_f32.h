@@ -6,9 +6,10 @@
 //     cast to fp32, P = exp(qk - max) in fp32, acc += P V);
 //   decode_attention (kernels/decode.py:84, 92-160) and
 //   speculative_decode_attention (kernels/speculative_decode.py:91-175):
-//     q, k, v in fp32, weights in fp32 (packed-head mode, KArgs::pack_m).
+//     q, k, v in fp32, weights in fp32 (packed-head mode, KArgs::pack_m), at
+//     head dims 16, 32 and 256 (64 and 128: fa2_kernel_decode_f32.h).
 // flash_attention_v2 rounds fp32 operands to fp16 (attention.py:547-633): it
-// runs the 16-bit kernels on fp16 copies, or the register-staged kernel of
+// runs the 16-bit kernels on fp16 operands, or the register-staged kernel of
 // fa2_device.h.
 //
 // Layout (one workgroup = 4 waves, 128 query rows, 32 per wave; KV tiles of

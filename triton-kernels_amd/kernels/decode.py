@@ -14,12 +14,12 @@ Same signature, assertion sequence and mode selection as the reference.
 The computation runs in ``libfa2.so`` (``fa2_decode_fwd``, include/fa2.h):
 the QH/KVH query heads that share a kv head are the rows of one work unit,
 so each K/V row is streamed from HBM once per kv head, and the KV sweep is
-split across workgroups with a log-sum-exp combine (the reference's split +
-merge, decode.py:22-200).  No CPU or PyTorch fallback.
+cut across workgroups with a log-sum-exp merge by the last of a unit's pieces
+(the reference's split + merge, decode.py:22-200).  No CPU or PyTorch fallback.
 
 Numerics: the reference loads every dtype into fp32 and computes in fp32
 (decode.py:84, 92-160).  fp32 tensors do the same here, on the fp32 MFMA
-(``v_mfma_f32_32x32x2_f32``: fp32 operands and softmax weights), so values
+(``v_mfma_f32_16x16x4_f32``: fp32 operands and softmax weights), so values
 past fp16's range stay finite.  fp16/bf16 tensors are exact in fp32 and run on
 the 16-bit MFMA with fp32 accumulation and fp32 softmax statistics; only P is
 rounded to the tensor type for the P.V product.  Both are within the
