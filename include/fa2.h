@@ -189,9 +189,9 @@ enum fa2_kernel {
 /* Bytes of device workspace fa2_fwd needs for `p` (0 is possible).
  * Replaces the reference's per-call torch.empty of running_sum/max/acc
  * (attention.py:852-864).  fp32 tensors with FA2_ARITH_REFERENCE at
- * head_dim 64/128 (dense, ragged) also hold fp16 copies of k and v, and of q where a
- * two-head kernel serves them, there,
- * as the reference rounds every fp32 operand to fp16.  Paged calls with one
+ * head_dim 64/128 (dense, ragged) also hold fp16 copies of q, k and v and
+ * one split's fp32 partials there, as the reference rounds every fp32 operand to
+ * fp16 (also where the kernel that serves them needs only k and v).  Paged calls with one
  * q-block per sequence and more two-head units than compute units hold the
  * partials of units their balanced walk cuts into pieces (4 * CUs * 128 *
  * (2 + head_dim) * 4 bytes).  Host-only: touches

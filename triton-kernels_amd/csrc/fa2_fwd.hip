@@ -500,14 +500,17 @@ int finish_plan(const fa2_params* p, Plan* pl) {
   off = (off + 255) & ~size_t(255);
   const size_t slots = pl->walk  ? static_cast<size_t>(2 * pl->grid_x)  // two pieces per workgroup
                        : pl->bal ? static_cast<size_t>(pl->bal_slots)
-                       : parts   ? static_cast<size_t>(splits) * pl->grid_x
+                       : parts || pl->conv ? static_cast<size_t>(splits) * pl->grid_x
                                  : 0;
   pl->off_ml = off;
   off += slots * pl->part_rows * 2 * sizeof(float);
   off = (off + 255) & ~size_t(255);
   pl->off_o = off;
   off += slots * pl->part_rows * pl->dim * sizeof(float);
-  // fp16 copies: q [B][Hq][Lq][D] or [Tq][Hq][D], k and v likewise
+  // fp16 copies: q [B][Hq][Lq][D] or [Tq][Hq][D], k and v likewise.  (The size
+  // told to callers holds q's copy and one split's partials for every such call,
+  // also where its kernel needs neither, so that it does not hang on which
+  // kernel serves the call.)
   const int64_t qrows = p->layout == FA2_LAYOUT_DENSE ? p->batch * p->q_len : p->q_len;
   const int64_t kvrows = p->layout == FA2_LAYOUT_DENSE ? p->batch * p->kv_len : p->kv_len;
   auto copy = [&](size_t& at, int64_t rows, int64_t heads) {
@@ -515,7 +518,7 @@ int finish_plan(const fa2_params* p, Plan* pl) {
     at = off;
     if (pl->conv) off += static_cast<size_t>(rows) * heads * p->head_dim * 2;
   };
-  copy(pl->off_cq, pl->pp ? qrows : 0, p->q_heads);
+  copy(pl->off_cq, qrows, p->q_heads);
   copy(pl->off_ck, kvrows, p->kv_heads);
   copy(pl->off_cv, kvrows, p->kv_heads);
   pl->total = off;
