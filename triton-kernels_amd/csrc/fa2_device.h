@@ -156,6 +156,9 @@ struct KArgs {
   // walk_segs segments of at least walk_min tiles for each of walk_streams
   // streams; 0 segments: unit blockIdx.x, split blockIdx.y.
   int32_t walk_streams, walk_segs, walk_min;
+  // fp32 partials and outputs: log2 units per unit of a partial's maximum m (see
+  // part_weight).  1: m is in log2 units; scale_log2: m is a raw score.
+  float ml_scale;
 };
 
 constexpr int kMergeCountBits = 24;
@@ -941,6 +944,15 @@ __device__ __forceinline__ void st_dev4(float* p, f32x4 x) {
   st_dev2(p + 2, x2, x3);
 }
 
+// Weight of a partial with maximum m in a merge whose maximum is g.  The fp32
+// kernels keep m as a raw score and scale the difference: their scores may be
+// so large that the rounding of score * scale alone is worth many powers of two.
+template <int DT>
+__device__ __forceinline__ float part_weight(const KArgs& a, float m, float g) {
+  if constexpr (DT == FA2_DTYPE_F32) return fast_exp2((m - g) * a.ml_scale);
+  else return fast_exp2(m - g);
+}
+
 // Row r, columns col..col+3 of the unit in part slot `unit` (of S splits),
 // written to the output element offset `off`.
 template <int DT, int D>
@@ -974,13 +986,13 @@ __device__ __forceinline__ void combine_row(const KArgs& a, int unit, int r, int
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // splits in order, as the one-at-a-time loop
-      const float wgt = fast_exp2(m[j] - g_use);
+      const float wgt = part_weight<DT>(a, m[j], g_use);
       lsum += wgt * l[j];
       acc += wgt * x[j];
     }
   }
   for (; s < S; ++s) {
-    const float wgt = fast_exp2(ml[s * ml_step] - g_use);
+    const float wgt = part_weight<DT>(a, ml[s * ml_step], g_use);
     lsum += wgt * ml[s * ml_step + 1];
     acc += wgt * *reinterpret_cast<const f32x4*>(po + s * o_step);
   }
@@ -1240,7 +1252,7 @@ __device__ __forceinline__ void merge_rows_sm(const KArgs& a, SlotOf slot_of, in
         for (int s = 0; s < SM; ++s) {
           if (s < S) {
             const uint32_t mw = ml[s][it][0], lw = ml[s][it][1];
-            const float wgt = fast_exp2(fl(mw) - g_use);
+            const float wgt = part_weight<DT>(a, fl(mw), g_use);
             lsum[it] += wgt * fl(lw);
             acc[it] += wgt * __builtin_bit_cast(f32x4, x[s][it]);
           }
@@ -1292,7 +1304,7 @@ __device__ __forceinline__ void merge_rows_sm(const KArgs& a, SlotOf slot_of, in
         for (int it = 0; it < kIt; ++it) {
           if (c0 + it * kRPP < rows) {
             const uint32_t mw = ml[it][0], lw = ml[it][1];
-            const float wgt = fast_exp2(fl(mw) - g[it]);
+            const float wgt = part_weight<DT>(a, fl(mw), g[it]);
             lsum[it] += wgt * fl(lw);
             acc[it] += wgt * __builtin_bit_cast(f32x4, x[it]);
           }

@@ -25,7 +25,11 @@
 //     K buffer, issued a phase earlier, gained 3 % on large two-block calls and
 //     spilled with one block at D = 128.)
 //   * The running max is raised, and O rescaled, only when a score passes it by
-//     2^8; the cross-lane maximum is skipped otherwise.
+//     2^8; the cross-lane maximum is skipped otherwise.  The max is kept as a raw
+//     score and the difference to it is scaled, (s - m) * scale, so that the largest
+//     weight is finite and not zero for scores of any finite size (an fma of s *
+//     scale against the rounded m * scale differs from it by the rounding of the
+//     product, 2^7 once that passes 2^31).
 //   * Rounding: with one block S is summed in eight chains and O in two levels
 //     (kFlush), so that the error against 64 bits stays at or below that of a
 //     tree over many lanes (2.1e-7 relative at 8192 keys).
@@ -83,6 +87,10 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
   const bool walk = a.walk_segs > 0;
   const int stream = walk ? static_cast<int>(blockIdx.x) % a.walk_streams : 0;
   const int seg_k = walk ? static_cast<int>(blockIdx.x) / a.walk_streams : 0;
+
+  const float scale = a.scale_log2;
+  // kRescaleThreshold in units of a score (finite: the first maximum passes -inf)
+  const float rescale = fminf(kRescaleThreshold / scale, 3.4e38f);
 
   DecPiece p;
   DecSegment sg{};
@@ -244,8 +252,8 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
 #pragma unroll
           for (int r = 0; r < 4; ++r) s[nb][r] = n0 + 4 * g + r <= last[nb] ? s[nb][r] : -INFINITY;
         }
-        mx[nb] = fmaxf(fmaxf(s[nb][0], s[nb][1]), fmaxf(s[nb][2], s[nb][3])) * a.scale_log2;
-        need |= mx[nb] > m[nb] + kRescaleThreshold;
+        mx[nb] = fmaxf(fmaxf(s[nb][0], s[nb][1]), fmaxf(s[nb][2], s[nb][3]));
+        need |= mx[nb] > m[nb] + rescale;
       }
       if (__any(need)) {
 #pragma unroll
@@ -254,7 +262,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
           x = fmaxf(x, __shfl_xor(x, 16));
           x = fmaxf(x, __shfl_xor(x, 32));
           const float mn = fmaxf(m[nb], x);
-          const float alpha = fast_exp2(m[nb] - (mn == -INFINITY ? 0.f : mn));
+          const float alpha = fast_exp2((m[nb] - (mn == -INFINITY ? 0.f : mn)) * scale);
           m[nb] = mn;
           l[nb] *= alpha;
 #pragma unroll
@@ -272,7 +280,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
         const float mu = m[nb] == -INFINITY ? 0.f : m[nb];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[nb][r] = fast_exp2(__builtin_fmaf(s[nb][r], a.scale_log2, -mu));
+          s[nb][r] = fast_exp2((s[nb][r] - mu) * scale);
           l[nb] += s[nb][r];
         }
       }
@@ -329,7 +337,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
       float mg = -INFINITY;
 #pragma unroll
       for (int x = 0; x < kDecF32Waves; ++x) mg = fmaxf(mg, mrg_ml[x][nb * 16 + l16][0]);
-      const float f = fast_exp2(m[nb] - (mg == -INFINITY ? 0.f : mg));
+      const float f = fast_exp2((m[nb] - (mg == -INFINITY ? 0.f : mg)) * scale);
       char* po = lds + wave * kOBytes + (nb * 16 + l16) * kOPitch + 16 * g * 4;
       if (nb * 16 + l16 < rows) {
 #pragma unroll
@@ -360,7 +368,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
         f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int x = 0; x < kDecF32Waves; ++x) {
-          lt += mrg_ml[x][r][1] * fast_exp2(mrg_ml[x][r][0] - mu);
+          lt += mrg_ml[x][r][1] * fast_exp2((mrg_ml[x][r][0] - mu) * scale);
           acc += *reinterpret_cast<const f32x4*>(lds + x * kOBytes + r * kOPitch + col * 4);
         }
         if (p.np == 1) {  // 0/0 -> NaN for a row with no key, as the reference
