@@ -40,7 +40,8 @@ def check_one_hot(q, k, v, out, off):
     sure = torch.ones_like(top[..., 0], dtype=torch.bool)
     if N > 1:
         sure = top[..., 0] - top[..., 1] > err + 150 * D ** 0.5
-    assert sure.double().mean() > 0.9
+    # (about one row in 700 falls below the bound at D = 256; cases have as few as 4)
+    assert sure.double().mean() > 0.5
     expect = torch.gather(v, 1, at[..., :1].expand(-1, -1, D))
     assert torch.isfinite(out).all()
     assert torch.equal(out[sure], expect[sure])
@@ -67,3 +68,24 @@ def test_fp32_decode_of_large_scores(layout, D, heads, M, size, splits):
     for b, out in enumerate(run(case, layout, num_splits=splits)):
         k = case.ks[b]
         check_one_hot(case.qs[b], k, case.vs[b], out, k.shape[0] - M if M > 1 else k.shape[0])
+
+
+@pytest.mark.parametrize("splits", [0, 3], ids=["auto", "forced"])
+@pytest.mark.parametrize("heads,M", [((4, 4), 1), ((8, 2), 8)], ids=["rows1", "rows32"])
+@pytest.mark.parametrize("D", [16, 32, 256])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_fp32_decode_of_large_scores_other_head_dims(layout, D, heads, M, splits):
+    test_fp32_decode_of_large_scores(layout, D, heads, M, 1e5, splits)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [16, 64, 128, 256])
+def test_flash_attention_v1_of_large_scores(D, causal):
+    from kernels import flash_attention_v1
+    g = torch.Generator().manual_seed(8300 + D)
+    q, k, v = (torch.randn((2, h, 300, D), generator=g) for h in (4, 2, 2))
+    q, k = q * 1e5, k * 1e5
+    out = flash_attention_v1(q.cuda(), k.cuda(), v.cuda(), is_causal=causal).cpu()
+    for b in range(2):
+        check_one_hot(q[b], k[b].transpose(0, 1), v[b].transpose(0, 1), out[b],
+                      0 if causal else 300)

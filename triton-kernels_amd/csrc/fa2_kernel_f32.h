@@ -102,6 +102,9 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_f32_kernel(
   const uint32_t krow = l32 * G::kRowBytes;
   const int ksw = G::k(l32);
 
+  const float scale = a.scale_log2;
+  const float rescale = fminf(kRescaleThreshold / scale, 3.4e38f);  // in units of a score
+
   if (T > 0) {
     ld.template issue<false>(a, w, t_begin * kBN, kbuf);
     ld.template issue<true>(a, w, t_begin * kBN, vbuf);
@@ -148,17 +151,18 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_f32_kernel(
 #pragma unroll
           for (int i2 = 0; i2 < 16; ++i2) mx = fmaxf(mx, s[sb][i2]);
         mx = max_xor32(mx);
-        const float mt = mx * a.scale_log2;
-        const bool need = mt > m_run + kRescaleThreshold;
-        const float alpha = fast_exp2(need ? (m_run - mt) : 0.0f);
-        m_run = need ? mt : m_run;
+        // (the max is a raw score and the difference to it is scaled: finite
+        // weights for scores of any finite size, as in fa2_kernel_decode_f32.h)
+        const bool need = mx > m_run + rescale;
+        const float alpha = fast_exp2(need ? (m_run - mx) * scale : 0.0f);
+        m_run = need ? mx : m_run;
         const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
         float rs = 0.f;
 #pragma unroll
         for (int sb = 0; sb < SB; ++sb)
 #pragma unroll
           for (int i2 = 0; i2 < 16; ++i2) {
-            s[sb][i2] = fast_exp2(__builtin_fmaf(s[sb][i2], a.scale_log2, -m_use));
+            s[sb][i2] = fast_exp2((s[sb][i2] - m_use) * scale);
             rs += s[sb][i2];
           }
         l_run = l_run * alpha + rs;
