@@ -102,10 +102,11 @@ def test_walk_one_sequence_in_many_pieces_16bit(layout, n):
     assert all(torch.equal(x, y) for x, y in zip(a, run(case, layout, decode=True)))
 
 
-# ---- short units, which stay whole: up to 12 tiles of 64 keys in 16 bits, 6 in fp32 ----
+# ---- short units, which stay whole: up to 12 tiles of 64 keys in 16 bits, 4 in fp32 (6: cut) ----
 
 @pytest.mark.parametrize("dt,top", [(torch.bfloat16, 12 * 64), (torch.float16, 12 * 64),
-                                    (torch.float32, 6 * 64)], ids=["bf16", "fp16", "fp32"])
+                                    (torch.float32, 6 * 64), (torch.float32, 4 * 64)],
+                         ids=["bf16", "fp16", "fp32", "fp32-4"])
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("past", [0, 1], ids=["whole", "cut"])
 def test_short_units_stay_whole(layout, dt, top, past):
@@ -114,3 +115,33 @@ def test_short_units_stay_whole(layout, dt, top, past):
     lens = [top + past] * 5 if layout == "dense" else [top + past, 0, 1, 64, 65, 300, 17, 0, 130]
     case = make_decode_case(len(lens), 128, 128, 64, 2, dt, layout, seed=5700, ctx_lens=lens)
     check(case, layout, run(case, layout))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("QH,KVH,n", [(5, 5, 200), (12, 12, 700), (48, 48, 230), (3, 3, 1900)])
+def test_streams_that_do_not_divide_the_grid(layout, dt, QH, KVH, n):
+    """Whole units that go round all workgroups (fp32: also those past the
+    streams' segments), and units long enough to be cut."""
+    lens = [n] * 11 if layout == "dense" else [max(0, n - 37 * i) for i in range(11)]
+    case = make_decode_case(len(lens), QH, KVH, 64, 1, dt, layout, seed=5750 + KVH, ctx_lens=lens)
+    check(case, layout, run(case, layout, decode=True))
+
+
+# ---- fp32 calls of many units: four-wave workgroups, blocks of 64 rows ----
+
+@pytest.mark.parametrize("heads,M", [((6, 6), 1), ((24, 6), 4), ((8, 1), 8), ((33, 1), 1),
+                                     ((16, 1), 8), ((18, 2), 5)],
+                         ids=["rows1", "rows16", "rows64", "rows33", "rows128", "rows45"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("splits", [0, 3])
+def test_many_units_f32(layout, D, heads, M, splits):
+    """Over 3/2 units per CU with up to 16 rows, and over 1/2 per CU of 64 rows."""
+    QH, KVH = heads
+    B = 130 if QH // KVH * M > 16 else 70
+    lens = [330] * B if layout == "dense" else [LENS[:-1][i % 10] if i % 13 else 700 + i
+                                               for i in range(B)]
+    case = make_decode_case(B, QH, KVH, D, M, torch.float32, layout, seed=5850 + M, causal=M > 1,
+                            ctx_lens=lens)
+    check(case, layout, run(case, layout, num_splits=splits))

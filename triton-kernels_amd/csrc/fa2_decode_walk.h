@@ -3,25 +3,22 @@
 //
 // A call's units are (sequence, kv head, q-block).  The kv heads and
 // q-blocks form a.walk_streams streams; stream s holds the units (b, s) of
-// all sequences in order, unit b weighing max(1, ceil(Lk_b / TK)) tiles of TK
-// keys (64, or the 128 of one ring slot).
-// The grid is walk_streams * walk_segs workgroups: workgroup g takes stream
-// g % walk_streams and segment k = g / walk_streams of it, tiles [k C, (k +
-// 1) C) with C = ceil(total / walk_segs), at least a.walk_min.  The kv heads
-// of a sequence are therefore read at about the same time (paged rows hold
-// all of them side by side), whatever the spread of the lengths every
-// workgroup streams at most C tiles, and no plan kernel is launched.  A unit
-// that a segment boundary cuts runs as pieces whose partials the last one
-// to finish merges, in piece order (merge_count, merge_rows_at): the cut
-// points follow from the lengths alone, so results do not depend on timing.
+// all sequences in order, unit b weighing max(1, ceil(Lk_b / TK)) tiles of
+// TK = 64 keys.  The grid starts with walk_streams * walk_segs workgroups:
+// workgroup g takes stream g % walk_streams and segment k = g / walk_streams of
+// it, tiles [k C, (k + 1) C) with C = ceil(total / walk_segs), at least
+// a.walk_min.  The kv heads of a sequence are therefore read at about the same
+// time (paged rows hold all of them side by side), whatever the spread of the
+// lengths every workgroup streams at most C tiles, and no plan kernel is
+// launched.  A unit that a segment boundary cuts runs as pieces whose partials
+// the last one to finish merges, in piece order (merge_count, merge_pieces): the
+// cut points follow from the lengths alone, so results do not depend on timing.
 //
-// When no unit has more than WHOLE tiles, cutting one costs more than it saves:
-// workgroup (s, k) then takes the whole units k, k + walk_segs, ... of its stream.
-// Measured on MI355X (us per call, always cut / whole up to 6 / up to 12 tiles):
-// 16-bit, 3 x 133 keys 16.6 / 8.2 / 8.1, 4 x 517 18.3 / 18.6 / 10.0, 64 x 16-600
-// 28.6 / 28.8 / 21.6; fp32, 8 x 20-300 keys 17.9 / 15.4 / 15.3, 4 x 517 16.9 /
-// 17.3 / 22.0.  The 16-bit kernel takes 12, the fp32 kernel, whose tiles take
-// longer, 6.
+// Whole units: cutting one costs its partials' round trip, about walk_whole tiles
+// of a workgroup's time.  So when no unit has more than walk_short tiles, or the
+// longest workgroup would take no more than walk_whole tiles beyond C with whole
+// units, workgroup g takes the whole units g, g + gridDim.x, ... of the call, in
+// the order (sequence, stream).
 //
 // Without a walk (walk_segs == 0, a forced split count) workgroup (x, y) runs
 // split y of unit x.
@@ -32,7 +29,7 @@
 namespace fa2 {
 
 // Sequences one lane of the locating wave adds up at most.
-constexpr int kWalkMaxPer = 64;
+constexpr int kWalkMaxPer = 1024;
 
 // One piece of a unit for this workgroup.
 struct DecPiece {
@@ -97,26 +94,28 @@ struct DecSegment {
   int j, us, s0, s1, C;
 };
 
-// By one wave: the segment of workgroup (stream, k) into *sh (LDS).
-template <int MODE, int TK, int WHOLE>
+// Whether units of up to `longest` tiles stay whole, walk_rounds of them per
+// workgroup, rather than C tiles of cut ones.
+__device__ __forceinline__ bool walk_keep_whole(const KArgs& a, int longest, int C) {
+  return longest <= a.walk_short || a.walk_rounds <= (C + a.walk_whole) / longest;
+}
+
+// By one wave: segment k of a stream into *sh (LDS); k >= walk_segs: empty.
+template <int MODE, int TK>
 __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* sh) {
   const int lane = threadIdx.x & 63;
   const int segs = a.walk_segs;
   if constexpr (MODE == FA2_LAYOUT_DENSE) {
     if (lane == 0) {
       const int W = walk_weight<TK>(a.kv_len);
-      if (W <= WHOLE) {
+      const int total = W * a.batch;
+      const int C = max((total + segs - 1) / segs, a.walk_min);
+      if (walk_keep_whole(a, W, C)) {
         *sh = DecSegment{k, 0, 0, 0, 0};
         return;
       }
-      const int total = W * a.batch;
-      const int C = max((total + segs - 1) / segs, a.walk_min);
       const int s0 = min(k * C, total);
-      sh->C = C;
-      sh->s0 = s0;
-      sh->s1 = min(s0 + C, total);
-      sh->j = s0 / W;
-      sh->us = (s0 / W) * W;
+      *sh = DecSegment{s0 / W, (s0 / W) * W, s0, min(s0 + C, total), C};
     }
     return;
   }
@@ -128,6 +127,10 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
     sum += W;
     longest = max(longest, W);
   }
+  if (!__any(longest > a.walk_short)) {
+    if (lane == 0) *sh = DecSegment{k, 0, 0, 0, 0};
+    return;
+  }
   int incl = sum;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -135,12 +138,12 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
     if (lane >= d) incl += y;
     longest = max(longest, __shfl_xor(longest, d));
   }
-  if (longest <= WHOLE) {
+  const int total = __shfl(incl, 63);
+  const int C = max((total + segs - 1) / segs, a.walk_min);
+  if (walk_keep_whole(a, longest, C)) {
     if (lane == 0) *sh = DecSegment{k, 0, 0, 0, 0};
     return;
   }
-  const int total = __shfl(incl, 63);
-  const int C = max((total + segs - 1) / segs, a.walk_min);
   const int s0 = min(k * C, total);
   const int excl = incl - sum;
   if (excl <= s0 && s0 < incl) {  // one lane, or none past the end
@@ -150,17 +153,9 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
       if (s0 < us + W) break;
       us += W;
     }
-    sh->j = j;
-    sh->us = us;
-    sh->s0 = s0;
-    sh->s1 = min(s0 + C, total);
-    sh->C = C;
+    *sh = DecSegment{j, us, s0, min(s0 + C, total), C};
   } else if (lane == 0 && s0 >= total) {
-    sh->j = a.batch;
-    sh->us = total;
-    sh->s0 = total;
-    sh->s1 = total;
-    sh->C = C;
+    *sh = DecSegment{a.batch, total, total, total, C};
   }
 }
 
@@ -197,14 +192,32 @@ __device__ __forceinline__ int walk_next(const KArgs& a, const DecSegment& g, in
   return b + (g.C == 0 ? a.walk_segs : 1);
 }
 
+// The sequence and stream of the next piece where whole units go round all
+// workgroups: the unit gridDim.x = walk_dj * walk_streams + walk_ds further.
+__device__ __forceinline__ void walk_next_unit(const KArgs& a, const DecSegment& g, int& j,
+                                               int& stream) {
+  if (g.C != 0) {
+    ++j;
+    return;
+  }
+  j += a.walk_dj;
+  stream += a.walk_ds;
+  if (stream >= a.walk_streams) {
+    stream -= a.walk_streams;
+    ++j;
+  }
+}
+
 // Split blockIdx.y of unit blockIdx.x (no walk); false: no such unit.
 template <int MODE, int TK>
 __device__ __forceinline__ bool split_piece(const KArgs& a, DecPiece& p) {
   p.w = decode_work<MODE>(a, blockIdx.x);
   if (!p.w.valid) return false;
-  const int S = a.num_splits;
-  const int split = blockIdx.y;
   const int tiles = (p.w.Lk + TK - 1) / TK;
+  // (splits past the unit's tiles would have none: they are not counted)
+  const int S = a.merge_ctr ? min(a.num_splits, max(tiles, 1)) : a.num_splits;
+  const int split = blockIdx.y;
+  if (split >= S) return false;
   p.t0 = (tiles * split) / S;
   p.T = (tiles * (split + 1)) / S - p.t0;
   p.np = S;

@@ -155,7 +155,9 @@ struct KArgs {
   // Decode kernels, automatic splits: the balanced walk (fa2_decode_walk.h),
   // walk_segs segments of at least walk_min tiles for each of walk_streams
   // streams; 0 segments: unit blockIdx.x, split blockIdx.y.
-  int32_t walk_streams, walk_segs, walk_min;
+  int32_t walk_streams, walk_segs, walk_min, walk_whole, walk_short;
+  int32_t walk_rounds;       // whole units per workgroup at most
+  int32_t walk_dj, walk_ds;  // gridDim.x / walk_streams, gridDim.x % walk_streams
   // fp32 partials and outputs: log2 units per unit of a partial's maximum m (see
   // part_weight).  1: m is in log2 units; scale_log2: m is a raw score.
   float ml_scale;

@@ -79,10 +79,22 @@ constexpr int64_t kF32DecodeMinTiles = 32;
 // keys Hq32/Hkv8 D128 23.5 / 23.7 / 31.2, 4 of 100-900 keys 18.9 / 21.7 / 28.7,
 // 4 x 1023 dense 19.5 / 21.2 / 26.9; calls that fill the GPU do not change.
 constexpr int64_t kDecF32MinTiles = 2;
-// ... and the 16-bit wave kernel's (us per call at 1 / 2 / 4 / 8 tiles, host
-// included: 4 x 1023 dense D128 19.4 / 18.8 / 18.9 / 19.9, one sequence of 8000
-// 21.4 / 20.7 / 20.9 / 21.5)
-constexpr int64_t kDecMinTiles = 2;
+// ... and the 16-bit wave kernel's: 4 of 64 keys are one 32-key tile for each wave
+// at D128.  Measured, kernel time in us at 1 / 2 / 4 / 8 tiles, D128: one sequence
+// of 8192 keys Hq16/Hkv1 29 / 19 / 14.5 / 13.4, 4 x 2048 16 / 12.5 / 11.3 / 11.7,
+// 4 x 2048 Hq32/Hkv8 15.2 / 15.1 / 15.4 / 15.4, 64 x 500-1500 the same.
+constexpr int64_t kDecMinTiles = 4;
+// tiles of the call per workgroup of the walks at least
+constexpr int64_t kWalkGridTiles = 2;
+// Whole units of the walks (KArgs::walk_whole, walk_short), in KV tiles of 64 keys.
+// Measured on MI355X, kernel time in us, cut / whole.  16 bits, D64: 4 x 500-1500
+// keys Hkv8 25 / 10, 16 x 500-1500 Hkv8 22 / 15.5, 16 x 2048 Hkv1 15 / 12, 64 x
+// 2000-6000 Hkv8 111 / 119.  D128: 4 x 500-1500 Hkv8 21 / 15, 16 x 500-1500
+// Hkv8 21.6 / 23.5, 16 x 2048 Hkv4 18 / 24, 1 x 2048 Hkv96 24 / 29, 300 x 600-768
+// Hkv1 30 / 27.  fp32, D128: 1 x 500 Hkv4 12.7 / 18, 4 x 500 Hkv8 14 / 18, 33 x
+// 330-384 Hkv8 34 / 38.
+constexpr int64_t kWholeIdle = 24, kWholeBusy = 12, kWholeShort = 12;
+constexpr int64_t kWholeF32 = 2, kWholeShortF32 = 4;
 
 // byte offset of the kXcds claim counters after the work list's item count
 // (within the 256 bytes reserved there; a cache line of their own)
@@ -138,6 +150,7 @@ struct Plan {
   bool dec;         // packed fp16/bf16: the decode kernel
   bool f32;         // fp32 arithmetic: the fp32-MFMA kernel
   bool decf32;      // packed fp32 at head_dim 64/128: the fp32 decode kernel
+  bool dec4;        // ... workgroups of four waves, two per CU
   bool conv;        // fp32 tensors with the reference's fp16 rounding: fp16 copies in the
                     // workspace, the 16-bit kernels with fp32 output
   bool plan;        // ragged/paged: the plan kernel orders the work list
@@ -148,7 +161,7 @@ struct Plan {
   bool bal;         // paged: the two-head kernel's balanced walk (pp_bal_locate)
   int64_t bal_slots;  // ... its part slots (4 per workgroup)
   bool walk;          // decode: the balanced walk (fa2_decode_walk.h)
-  int64_t walk_streams, walk_segs, walk_min;
+  int64_t walk_streams, walk_segs, walk_min, walk_whole, walk_short;
   int64_t max_wgs;  // cap on the persistent grid (0: none)
   uint32_t pool_bytes_k, pool_bytes_v;
   size_t off_work, off_count, off_ml, off_o, off_ctr, off_cq, off_ck, off_cv, total;
@@ -498,7 +511,7 @@ int finish_plan(const fa2_params* p, Plan* pl) {
   else if (pl->fold || pl->bal)
     off += static_cast<size_t>(pl->grid_x) * sizeof(uint64_t);
   off = (off + 255) & ~size_t(255);
-  const size_t slots = pl->walk  ? static_cast<size_t>(2 * pl->grid_x)  // two pieces per workgroup
+  const size_t slots = pl->walk  ? static_cast<size_t>(2 * pl->walk_streams * pl->walk_segs)  // two cut pieces per workgroup
                        : pl->bal ? static_cast<size_t>(pl->bal_slots)
                        : parts || pl->conv ? static_cast<size_t>(splits) * pl->grid_x
                                  : 0;
@@ -540,14 +553,30 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   pl->dec = p->dtype != FA2_DTYPE_F32 && fast_dim(p->head_dim);
   pl->f32 = p->dtype == FA2_DTYPE_F32;  // decode's reference computes fp32 in fp32
   pl->conv = false;
-  // fp32 at head_dim 64/128: the fp32 decode kernel, blocks of 16 or 32 rows
-  // (four 16-row blocks' accumulators do not fit its registers)
+  // fp32 at head_dim 64/128: the fp32 decode kernel, blocks of 16 or 32 rows, or of
+  // 64 at head_dim 64 (at 128 their accumulators do not fit its registers) where
+  // they give every other CU a unit: each block reads all of its keys.  Measured on
+  // MI355X, D64, us per call, 32 / 64 rows: 64 sequences of 2000-6000 keys, 4 kv
+  // heads x 128 rows 430 / 350 (512 blocks), 16 of 500-1500, 8 x 64 rows 44 / 44
+  // (128), 4 of 500-1500, 8 x 64 rows 21 / 26 (32).
   pl->decf32 = pl->f32 && (p->head_dim == 64 || p->head_dim == 128);
-  pl->block_rows =
-      pl->dec ? kDecRows : (pl->decf32 ? (pl->rows <= 16 ? 16 : 32) : kBM);
+  const int64_t cus = query_device ? cu_count_current_device() : 256;
+  const bool rows64 = pl->dim == 64 && pl->rows > 32 &&
+                      2 * cdiv(pl->rows, 64) * p->batch * p->kv_heads >= cus;
+  pl->block_rows = pl->dec      ? kDecRows
+                   : !pl->decf32 ? kBM
+                                 : (pl->rows <= 16 ? 16 : rows64 ? 64 : 32);
   const int64_t nqb = cdiv(pl->rows, pl->block_rows);
   pl->work_ub = nqb * p->batch;
   pl->npairs = pl->work_ub * p->kv_heads;
+  // Single 16-row blocks, automatic splits, at least three units for every two CUs:
+  // two workgroups of four waves per CU, so that one streams while the other
+  // starts or merges a unit.  Measured on MI355X, us per call, eight waves / four:
+  // 64 x 50-150 keys Hq40/Hkv40 D128 98 / 81, 256 x 500-1500 Hq8/Hkv8 D64 252 /
+  // 230, 64 x 2000-6000 Hq8/Hkv8 D128, 8 drafts 361 / 364.  With fewer units the
+  // halves of a CU only double the partials: 4 x 32768 keys Hq16/Hkv1 D64 27 / 49.
+  pl->dec4 = pl->decf32 && pl->block_rows == 16 && p->num_splits == 0 &&
+             2 * pl->npairs >= 3 * cus;
   pl->grid_x = cdiv(pl->npairs, kXcds) * kXcds;
   if (pl->grid_x > INT32_MAX || pl->npairs > INT32_MAX) return FA2_ERR_TOO_LARGE;
   pl->pp = false;
@@ -556,16 +585,12 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   pl->grid_pp = 0;
   int splits = p->num_splits;
   if (splits == 0) {
-    const int64_t cus = query_device ? cu_count_current_device() : 256;
-    // The decode kernel holds a CU alone: one workgroup per CU, >= 8 tiles
-    // per split to keep its LDS ring in steady state (measured on MI355X:
-    // 128 units of 128 tiles run best at 2 splits, 512 units at 1).  The
-    // fp32 kernel (two workgroups per CU, no deep K/V pipeline) is
-    // latency-bound: it wants several rounds of workgroups, each sweeping
-    // >= 32 tiles (measured on MI355X, fp32 decode, us per call at 1 / 2 /
-    // 4 / 8 workgroups per CU and >= 8 tiles: d1 (128 units of 128 tiles)
-    // 338 / 180 / 187 / 204 at 2 / 4 / 8 / 16 splits; d2 (512 units, up to
-    // 128 tiles) 1730 / 1731 / 1148 / 1105 at 1 / 1 / 2 / 4 splits).
+    // The ring kernel holds a CU alone: one workgroup per CU, >= 8 tiles per split
+    // to keep its LDS ring in steady state (measured on MI355X: 128 units of 128
+    // tiles run best at 2 splits, 512 units at 1).  The fp32 kernel of the other
+    // head dims (two workgroups per CU, one at 256, no deep K/V pipeline) is
+    // latency-bound: it wants several rounds of workgroups, each sweeping >= 32
+    // tiles.  (Where the walks run, below, they replace this count.)
     const int64_t target = pl->dec ? cus : cus * kF32DecodeWgsPerCu;
     const int64_t min_tiles = pl->dec ? 8 : kF32DecodeMinTiles;
     const int64_t tiles = cdiv(kv_upper_bound(p), kBN);
@@ -588,9 +613,9 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   // was 7 % of the step.)
   pl->plan = p->layout != FA2_LAYOUT_DENSE;
   pl->dev_splits = false;
-  const int64_t resident = pl->dec ? 1 : (pl->dim > 128 ? 1 : 2);  // workgroups per CU
+  const int64_t resident = pl->dec || pl->decf32 || pl->dim > 128 ? 1 : 2;  // workgroups per CU
   if (pl->plan && (pl->dec || pl->f32) && query_device &&
-      pl->grid_x * splits <= cu_count_current_device() * resident)
+      pl->grid_x * splits <= cus * resident)
     pl->plan = false;
   // The decode kernel merges its own splits: the last split of a unit to
   // finish combines the unit's partials, so no combine launch follows.
@@ -605,17 +630,20 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   // ring, 212-226 waves), at 4 rows the waves are faster (207 -> 189).
   const bool wave = pl->dec && pl->rows <= kDwRows && p->decode_spin_cap == 0;
   if ((pl->decf32 || wave) && p->num_splits == 0 && p->batch <= 64 * kWalkMaxPer) {
-    const int64_t cus = query_device ? cu_count_current_device() : 256;
+    const int64_t wgs = cus * (pl->dec4 ? 2 : 1);
     const int64_t streams = p->kv_heads * nqb;
     const int64_t min_tiles = pl->dec ? kDecMinTiles : kDecF32MinTiles;
     const int64_t tiles = cdiv(kv_upper_bound(p), kBN) + 1;
     const int64_t total = p->layout == FA2_LAYOUT_RAGGED ? tiles + p->batch : tiles * p->batch;
-    int64_t segs = std::max<int64_t>(1, cus / streams);
-    segs = std::min(segs, cdiv(total, min_tiles));
-    // (32-bit byte offsets into the part slots; see merge_pieces)
+    int64_t segs = std::max<int64_t>(1, wgs / streams);
+    segs = std::min(segs, cdiv(total, kWalkGridTiles));
+    // (32-bit tile counts, also where pages repeat and sequences are longer than
+    // the pool; 32-bit byte offsets into the part slots, see merge_pieces)
+    const int64_t longest =
+        p->layout == FA2_LAYOUT_PAGED && p->kv_len_max > 0 ? cdiv(p->kv_len_max, kBN) * p->batch : 0;
     const int64_t part_bytes = 2 * streams * segs * pl->part_rows * pl->dim * 4;
-    if (total < (int64_t(1) << 30) && part_bytes < (int64_t(1) << 31) &&
-        streams * p->batch <= INT32_MAX) {
+    if (std::max(total, longest) < (int64_t(1) << 30) && part_bytes < (int64_t(1) << 31) &&
+        streams * p->batch <= INT32_MAX / 2) {
       pl->walk = true;
       pl->walk_streams = streams;
       pl->walk_segs = segs;
@@ -624,7 +652,18 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
       pl->splits = 1;
       pl->fold = false;
       pl->grid_x = streams * segs;
+      // fp32: more workgroups, which only take whole units
+      if (pl->decf32) pl->grid_x = std::max(pl->grid_x, std::min(wgs, streams * p->batch));
       if (wave) pl->block_rows = kDwRows;
+      // What cutting costs in 16 bits, in tiles: more where few units leave most
+      // CUs idle and a tile is mostly latency, twice as many at head_dim 64, whose
+      // tiles are half the bytes.
+      const int64_t idle = std::max<int64_t>(0, pl->grid_x - streams * p->batch);
+      pl->walk_whole = pl->decf32 ? kWholeF32
+                                  : std::max(kWholeBusy * 128 / pl->dim,
+                                             (pl->dim == 64 ? 3 : 2) * kWholeIdle * idle /
+                                                 (2 * pl->grid_x));
+      pl->walk_short = pl->decf32 ? kWholeShortF32 : kWholeShort;
     }
   }
   return finish_plan(p, pl);
@@ -681,12 +720,15 @@ int launch_typed(KArgs a, const Plan& pl, hipStream_t st) {
   const dim3 grid(pl.grid_x, pl.splits);
   if constexpr (DT == FA2_DTYPE_F32 && (D == 64 || D == 128)) {
     if (pl.decf32) {
-      if (pl.block_rows == 16)
-        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 1>), grid, dim3(kDecF32Threads), 0, st,
-                           a);
-      else
-        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 2>), grid, dim3(kDecF32Threads), 0, st,
-                           a);
+      const dim3 block(pl.dec4 ? 256 : 512);
+      if (pl.dec4)
+        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 1, 4>), grid, block, 0, st, a);
+      else if (pl.block_rows == 16)
+        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 1, 8>), grid, block, 0, st, a);
+      else if (pl.block_rows == 32)
+        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 2, 8>), grid, block, 0, st, a);
+      else if constexpr (D == 64)
+        hipLaunchKernelGGL((fa2_decode_f32_kernel<D, MODE, 4, 8>), grid, block, 0, st, a);
       if (pl.splits > 1 && !pl.fold)
         hipLaunchKernelGGL((fa2_combine_kernel<DT, D, MODE>),
                            dim3(pl.grid_x, cdiv(pl.part_rows, kCombineRows<D>)), dim3(kThreads),
@@ -936,6 +978,13 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
   a.walk_streams = static_cast<int32_t>(pl.walk_streams);
   a.walk_segs = pl.walk ? static_cast<int32_t>(pl.walk_segs) : 0;
   a.walk_min = static_cast<int32_t>(pl.walk_min);
+  a.walk_whole = static_cast<int32_t>(pl.walk_whole);
+  a.walk_short = static_cast<int32_t>(pl.walk_short);
+  if (pl.walk) {
+    a.walk_dj = static_cast<int32_t>(pl.grid_x / pl.walk_streams);
+    a.walk_ds = static_cast<int32_t>(pl.grid_x % pl.walk_streams);
+    a.walk_rounds = static_cast<int32_t>(cdiv(pl.walk_streams * p->batch, pl.grid_x));
+  }
   a.pack_m = packed ? static_cast<int32_t>(p->q_len) : 0;
   a.dv = static_cast<int32_t>(p->head_dim);
   a.spin_cap = p->decode_spin_cap > 0 ? p->decode_spin_cap : kDecSpinCap;

@@ -7,8 +7,9 @@
 // rows; a key costs 4 * D * 16 NB FLOP of matrix work against 8 * D bytes.
 // With one block the MFMAs could take 17 TB/s of K/V, so the kernel is bound by
 // HBM; with two (17 to 32 rows) they take about 8.6, close to what HBM gives.
-//   * Workgroup = 8 waves, one per CU.  Each wave walks its own 16-key tiles
-//     (tile i of the workgroup's range to wave i % 8) with its own (m, l, O), so
+//   * Workgroup = 8 waves, one per CU (4, two per CU, in calls of many units of
+//     one block: make_plan_packed).  Each wave walks its own 16-key tiles
+//     (tile i of the workgroup's range to wave i % NW) with its own (m, l, O), so
 //     all four matrix cores work whatever the row count and no barrier stands
 //     between a load and its use.
 //   * S^T = K Q^T: the A operand of k-step (i, e) is K[key][16 i + 4 g + e] for
@@ -34,7 +35,12 @@
 //     (kFlush), so that the error against 64 bits stays at or below that of a
 //     tree over many lanes (2.1e-7 relative at 8192 keys).
 //   * The waves' states meet in LDS, added up by all threads in wave order; cut
-//     units merge through their partials (fa2_decode_walk.h).
+//     units merge through their partials (fa2_decode_walk.h).  The next piece's
+//     first tile and Q are loaded under the merge of a whole unit: 256 x 50-150 keys
+//     Hq32/Hkv32 D128 302 -> 276 us, with four-wave workgroups 220.
+//   * With several blocks per unit K and V stay in L2 for the others (no nt loads):
+//     64 x 2000-6000 keys, 8 kv heads x 128 rows D64 960 -> 830 us, with blocks of 64
+//     rows 700.
 //
 // Measured on MI355X, us per call, against a dot-product kernel on the VALU
 // (up to 8 rows) and 32x32x2 MFMAs with one 32-row block per wave (above):
@@ -48,17 +54,16 @@
 
 namespace fa2 {
 
-constexpr int kDecF32Waves = 8;
-constexpr int kDecF32Threads = 64 * kDecF32Waves;
-constexpr int kDecF32Whole = 6;  // units of up to this many 64-key tiles stay whole
+constexpr int kDecF32Waves = 8;  // waves of a CU: one workgroup, or two of four each
 
 __device__ __forceinline__ f32x4 mma16_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// NB: 16-row blocks of a unit (block_rows = 16 NB)
-template <int D, int MODE, int NB>
-__global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs a) {
+// NB: 16-row blocks of a unit (block_rows = 16 NB); NW: waves of a workgroup
+template <int D, int MODE, int NB, int NW>
+__global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kernel(KArgs a) {
+  constexpr int kThr = 64 * NW;
   constexpr int DJ = D / 16;  // 16-dim groups of K and Q: 4 MFMA k-steps each
   constexpr int DH = D / 64;  // 64-dim groups of V and O
   constexpr int R = 16 * NB;
@@ -71,10 +76,10 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
   // one wave's O, rows padded so that 16 lanes write 16 rows conflict-free
   constexpr int kOPitch = (D + 4) * 4;
   constexpr int kOBytes = R * kOPitch;
-  constexpr int kLds = kDecF32Waves * kOBytes;  // (Q first, then every wave's O)
-  static_assert(kLds >= kQBytes && kLds >= kMergePieceBytes<kDecF32Threads>, "LDS areas");
+  constexpr int kLds = NW * kOBytes;  // (Q first, then every wave's O)
+  static_assert(kLds >= kQBytes && kLds >= kMergePieceBytes<kThr>, "LDS areas");
   __shared__ __attribute__((aligned(16))) char lds[kLds];
-  __shared__ float mrg_ml[kDecF32Waves][R][2];
+  __shared__ float mrg_ml[NW][R][2];
   __shared__ DecSegment seg_sh;
   __shared__ int merge_flag;
 
@@ -85,7 +90,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
   const int g = lane >> 4;
   const bool causal = a.mask != FA2_MASK_NONE;
   const bool walk = a.walk_segs > 0;
-  const int stream = walk ? static_cast<int>(blockIdx.x) % a.walk_streams : 0;
+  int stream = walk ? static_cast<int>(blockIdx.x) % a.walk_streams : 0;
   const int seg_k = walk ? static_cast<int>(blockIdx.x) / a.walk_streams : 0;
 
   const float scale = a.scale_log2;
@@ -94,76 +99,77 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
 
   DecPiece p;
   DecSegment sg{};
-  int j = 0, us = 0;
   if (walk) {
-    if (wave == 0) walk_locate<MODE, kBN, kDecF32Whole>(a, seg_k, &seg_sh);
+    if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
     __syncthreads();
     sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
     sg.us = __builtin_amdgcn_readfirstlane(seg_sh.us);
     sg.s0 = __builtin_amdgcn_readfirstlane(seg_sh.s0);
     sg.s1 = __builtin_amdgcn_readfirstlane(seg_sh.s1);
     sg.C = __builtin_amdgcn_readfirstlane(seg_sh.C);
-    j = sg.j;
-    us = sg.us;
-    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, us, p)) return;
+    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, sg.j, sg.us, p)) return;
   } else if (!split_piece<MODE, kBN>(a, p)) {
     return;
   }
 
-  for (;;) {
-    const Work& w = p.w;
-    const int row0 = w.qblk * R;
-    const int rows = min(w.Lq - row0, R);
-    const int k_begin = p.t0 * kBN;
-    const int k_end = min((p.t0 + p.T) * kBN, w.Lk);
+  // The piece whose tiles are being loaded: its sequence, keys, and this wave's
+  // next tile.
+  int b, k_end, n0;
+  const float *kbase, *vbase;
+  constexpr int kStep = 16 * NW;
+  // physical rows (in K and V) of key n, clamped to the range, and to the
+  // pool where its size is known (no read outside the allocation)
+  auto row_of = [&](const int32_t* table, int64_t stride, int n) -> int {
+    n = max(min(n, k_end - 1), 0);
+    if constexpr (MODE == FA2_LAYOUT_PAGED) {
+      const int pidx = a.page_shift >= 0 ? n >> a.page_shift : n / a.page_size;
+      const int row = table[b * stride + pidx] * a.page_size + (n - pidx * a.page_size);
+      return a.kv_len > 0 ? min(max(row, 0), a.kv_len - 1) : row;
+    } else {
+      return n;
+    }
+  };
+  auto krow_of = [&](int n) { return row_of(a.k_table, a.k_table_stride, n); };
+  auto vrow_of = [&](int n) { return row_of(a.v_table, a.v_table_stride, n); };
 
-    // physical rows (in K and V) of key n, clamped to the range, and to the
-    // pool where its size is known (no read outside the allocation)
-    auto in_pool = [&](int row) { return a.kv_len > 0 ? min(max(row, 0), a.kv_len - 1) : row; };
-    auto krow_of = [&](int n) -> int {
-      n = max(min(n, k_end - 1), 0);
-      if constexpr (MODE == FA2_LAYOUT_PAGED) {
-        const int pidx = a.page_shift >= 0 ? n >> a.page_shift : n / a.page_size;
-        return in_pool(a.k_table[w.b * a.k_table_stride + pidx] * a.page_size +
-                       (n - pidx * a.page_size));
-      } else {
-        return n;
-      }
-    };
-    auto vrow_of = [&](int n) -> int {
-      n = max(min(n, k_end - 1), 0);
-      if constexpr (MODE == FA2_LAYOUT_PAGED) {
-        const int pidx = a.page_shift >= 0 ? n >> a.page_shift : n / a.page_size;
-        return in_pool(a.v_table[w.b * a.v_table_stride + pidx] * a.page_size +
-                       (n - pidx * a.page_size));
-      } else {
-        return n;
-      }
-    };
-    const float* kbase = static_cast<const float*>(a.k) + w.k_base + 4 * g;
-    const float* vbase = static_cast<const float*>(a.v) + w.v_base + 4 * l16;
-
-    f32x4 kx[DJ], vx[4][DH];
-    auto load_k = [&](int row) {
-      const f32x4* kp = reinterpret_cast<const f32x4*>(kbase + static_cast<int64_t>(row) * a.k_ss);
+  f32x4 kx[DJ], vx[4][DH];
+  auto load_k = [&](int row) {
+    const f32x4* kp = reinterpret_cast<const f32x4*>(kbase + static_cast<int64_t>(row) * a.k_ss);
 #pragma unroll
-      for (int i = 0; i < DJ; ++i) kx[i] = __builtin_nontemporal_load(kp + 4 * i);
-    };
-    auto load_v = [&](int row16) {  // row16: the physical row of key lane % 16
+    for (int i = 0; i < DJ; ++i) kx[i] = NB > 1 ? kp[4 * i] : __builtin_nontemporal_load(kp + 4 * i);
+  };
+  auto load_v = [&](int row16) {  // row16: the physical row of key lane % 16
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = __shfl(row16, 4 * g + r);
-        const f32x4* vp =
-            reinterpret_cast<const f32x4*>(vbase + static_cast<int64_t>(row) * a.v_ss);
+    for (int r = 0; r < 4; ++r) {
+      const int row = __shfl(row16, 4 * g + r);
+      const f32x4* vp = reinterpret_cast<const f32x4*>(vbase + static_cast<int64_t>(row) * a.v_ss);
 #pragma unroll
-        for (int h = 0; h < DH; ++h) vx[r][h] = __builtin_nontemporal_load(vp + 16 * h);
-      }
-    };
-
-    // first tile's loads, then Q into LDS in fragment order
-    int n0 = k_begin + wave * 16;  // this wave's tile
-    constexpr int kStep = 16 * kDecF32Waves;
-    int krow = 0, vrow = 0;
+      for (int h = 0; h < DH; ++h) vx[r][h] = NB > 1 ? vp[16 * h] : __builtin_nontemporal_load(vp + 16 * h);
+    }
+  };
+  int krow = 0, vrow = 0;  // of the tile after the one loaded
+  constexpr int kQF = (NB * DJ * 64 + kThr - 1) / kThr;
+  f32x4 qx[kQF];  // Q in fragment order, on its way to LDS
+  // the first tile's and Q's loads of piece x
+  auto begin = [&](const DecPiece& x) {
+    b = x.w.b;
+    k_end = min((x.t0 + x.T) * kBN, x.w.Lk);
+    n0 = x.t0 * kBN + wave * 16;
+    kbase = static_cast<const float*>(a.k) + x.w.k_base + 4 * g;
+    vbase = static_cast<const float*>(a.v) + x.w.v_base + 4 * l16;
+    const int row0 = x.w.qblk * R;
+    const int rows = min(x.w.Lq - row0, R);
+    const float* qp = static_cast<const float*>(a.q) + x.w.q_base;
+#pragma unroll
+    for (int y = 0; y < kQF; ++y) {
+      const int f = tid + y * kThr;
+      const int fl = f & 63, fj = (f >> 6) % DJ, fn = (f >> 6) / DJ;
+      const int row = fn * 16 + (fl & 15);
+      qx[y] = f < NB * DJ * 64 && row < rows
+                  ? *reinterpret_cast<const f32x4*>(
+                        qp + static_cast<int64_t>(row0 + row) * a.q_ss + 16 * fj + 4 * (fl >> 4))
+                  : (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
     if (n0 < k_end) {
       krow = krow_of(n0 + l16);
       vrow = vrow_of(n0 + l16);
@@ -172,17 +178,24 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
       krow = krow_of(n0 + kStep + l16);
       vrow = vrow_of(n0 + kStep + l16);
     }
-    {
-      const float* qp = static_cast<const float*>(a.q) + w.q_base;
-      for (int f = tid; f < NB * DJ * 64; f += kDecF32Threads) {
-        const int fl = f & 63, fj = (f >> 6) % DJ, fn = (f >> 6) / DJ;
-        const int row = fn * 16 + (fl & 15);
-        const f32x4 x = row < rows ? *reinterpret_cast<const f32x4*>(
-                                         qp + static_cast<int64_t>(row0 + row) * a.q_ss + 16 * fj +
-                                         4 * (fl >> 4))
-                                   : (f32x4){0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<f32x4*>(lds + f * 16) = x;
-      }
+  };
+
+  begin(p);
+  for (;;) {
+    const Work& w = p.w;
+    const int row0 = w.qblk * R;
+    const int rows = min(w.Lq - row0, R);
+#pragma unroll
+    for (int y = 0; y < kQF; ++y) {
+      const int f = tid + y * kThr;
+      if (f < NB * DJ * 64) *reinterpret_cast<f32x4*>(lds + f * 16) = qx[y];
+    }
+    DecPiece next;
+    bool has_next = walk;
+    if (walk) {
+      int j = w.b;
+      walk_next_unit(a, sg, j, stream);
+      has_next = walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, p.us + p.W, next);
     }
     int last[NB];  // last visible key of this lane's row
 #pragma unroll
@@ -320,6 +333,10 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
         for (int e = 0; e < 4; ++e) o[0][h][e] += o2[h][e];
     }
 
+    // the next piece's first loads run under this one's merge (a cut unit's piece
+    // publishes its partials and counts first: both wait for all earlier loads)
+    if (has_next && p.np == 1) begin(next);
+
     // merge the waves: their (m, l), then every wave's O scaled to the common
     // max goes through LDS and all threads add up rows, in wave order
 #pragma unroll
@@ -336,7 +353,7 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
     for (int nb = 0; nb < NB; ++nb) {
       float mg = -INFINITY;
 #pragma unroll
-      for (int x = 0; x < kDecF32Waves; ++x) mg = fmaxf(mg, mrg_ml[x][nb * 16 + l16][0]);
+      for (int x = 0; x < NW; ++x) mg = fmaxf(mg, mrg_ml[x][nb * 16 + l16][0]);
       const float f = fast_exp2((m[nb] - (mg == -INFINITY ? 0.f : mg)) * scale);
       char* po = lds + wave * kOBytes + (nb * 16 + l16) * kOPitch + 16 * g * 4;
       if (nb * 16 + l16 < rows) {
@@ -359,15 +376,15 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
       const __amdgpu_buffer_rsrc_t ro = make_rsrc_uniform(a.part_o + slot * pr * D, pr * D * 4);
       constexpr int kTPR = D / 4;
       const int col = (tid % kTPR) * 4;
-      for (int r = tid / kTPR; r < rows; r += kDecF32Threads / kTPR) {
+      for (int r = tid / kTPR; r < rows; r += kThr / kTPR) {
         float mg = -INFINITY;
 #pragma unroll
-        for (int x = 0; x < kDecF32Waves; ++x) mg = fmaxf(mg, mrg_ml[x][r][0]);
+        for (int x = 0; x < NW; ++x) mg = fmaxf(mg, mrg_ml[x][r][0]);
         const float mu = mg == -INFINITY ? 0.f : mg;
         float lt = 0.f;
         f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int x = 0; x < kDecF32Waves; ++x) {
+        for (int x = 0; x < NW; ++x) {
           lt += mrg_ml[x][r][1] * fast_exp2((mrg_ml[x][r][0] - mu) * scale);
           acc += *reinterpret_cast<const f32x4*>(lds + x * kOBytes + r * kOPitch + col * 4);
         }
@@ -390,17 +407,16 @@ __global__ __launch_bounds__(kDecF32Threads, 1) void fa2_decode_f32_kernel(KArgs
       __syncthreads();
       if (merge_count(a, p.unit, p.np, &merge_flag)) {
         if (walk)
-          merge_pieces<FA2_DTYPE_F32, D, kDecF32Threads, R>(
+          merge_pieces<FA2_DTYPE_F32, D, kThr, R>(
               a, [&](int s) { return walk_slot(a, sg.C, p.us, stream, s); }, p.np, rows, w.o_base,
               row0, lds);
         else
-          merge_rows<FA2_DTYPE_F32, D, kDecF32Threads, R>(a, p.unit, p.np, rows, w.o_base, row0);
+          merge_rows<FA2_DTYPE_F32, D, kThr, R>(a, p.unit, p.np, rows, w.o_base, row0);
       }
     }
-    if (!walk) return;
-    j = walk_next(a, sg, j);
-    us = p.us + p.W;
-    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, us, p)) return;
+    if (!has_next) return;
+    if (p.np > 1) begin(next);
+    p = next;
     __syncthreads();  // the merge area becomes Q again
   }
 }

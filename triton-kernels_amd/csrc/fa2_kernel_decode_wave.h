@@ -41,7 +41,6 @@ namespace fa2 {
 
 constexpr int kDwWaves = 8;
 constexpr int kDwThreads = 64 * kDwWaves;
-constexpr int kDwWhole = 12;      // units of up to this many 64-key tiles stay whole
 constexpr int kDwTable = 512;     // block-table entries of a window (K and V each)
 constexpr int kDwRows = 16;       // rows of a unit at most
 // rows that pass through LDS at once beside the tiles in flight
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(kDwThreads, 1) void fa2_decode_wave_kernel(KArgs a)
   const int stream = static_cast<int>(blockIdx.x) % a.walk_streams;
   const int seg_k = static_cast<int>(blockIdx.x) / a.walk_streams;
 
-  if (wave == 0) walk_locate<MODE, kBN, kDwWhole>(a, seg_k, &seg_sh);
+  if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
   __syncthreads();
   DecSegment sg;
   sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
