@@ -310,14 +310,14 @@ __device__ __forceinline__ void merge_pieces(const KArgs& a, SlotOf slot_of, int
           mn = fmaxf(mn, fl(mw));
         }
         const float mu = mn == -INFINITY ? 0.f : mn;
-        const float al = part_weight<DT>(a, m[it], mu);
+        const float al = fast_exp2(m[it] - mu);
         l[it] *= al;
         acc[it] *= al;
         m[it] = mn;
 #pragma unroll
         for (int j = 0; j < kB; ++j) {
           const uint32_t mw = ml[j][it][0], lw = ml[j][it][1];
-          const float wgt = part_weight<DT>(a, fl(mw), mu);
+          const float wgt = fast_exp2(fl(mw) - mu);
           l[it] += wgt * fl(lw);
           acc[it] += wgt * __builtin_bit_cast(f32x4, x[j][it]);
         }
@@ -338,7 +338,7 @@ __device__ __forceinline__ void merge_pieces(const KArgs& a, SlotOf slot_of, int
       acc[0] = (f32x4){0.f, 0.f, 0.f, 0.f};
       for (int q = 0; q < groups; ++q) {
         const int o = tid + q * span * kTPR;
-        const float wgt = part_weight<DT>(a, sh[NT * 4 + o * 2], mu);
+        const float wgt = fast_exp2(sh[NT * 4 + o * 2] - mu);
         l[0] += wgt * sh[NT * 4 + o * 2 + 1];
         acc[0] += wgt * *reinterpret_cast<const f32x4*>(sh + o * 4);
       }

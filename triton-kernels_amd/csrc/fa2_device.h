@@ -158,9 +158,6 @@ struct KArgs {
   int32_t walk_streams, walk_segs, walk_min, walk_whole, walk_short;
   int32_t walk_rounds;       // whole units per workgroup at most
   int32_t walk_dj, walk_ds;  // gridDim.x / walk_streams, gridDim.x % walk_streams
-  // fp32 partials and outputs: log2 units per unit of a partial's maximum m (see
-  // part_weight).  1: m is in log2 units; scale_log2: m is a raw score.
-  float ml_scale;
 };
 
 constexpr int kMergeCountBits = 24;
@@ -261,6 +258,34 @@ __device__ __forceinline__ f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Running maximum of the fp32 kernels' rows: mu = s * scale, rounded, of a score s.
+// An exponent is fma(s, scale, -mu), rounded once; for the largest score that is the
+// rounding error of mu, worth many powers of two once mu is large (2^7 at 2^31), and
+// there it is taken off again: res (0 otherwise).
+struct Max32 {
+  float mu, res;
+};
+__device__ __forceinline__ Max32 max32_of(float s, float scale) {
+#pragma clang fp contract(off)
+  const float mu = s * scale;
+  const float r = __builtin_fmaf(s, scale, -mu);
+  const float x = __builtin_fabsf(mu);
+  return {mu, x > 1048576.f && x < INFINITY ? r : 0.f};
+}
+// log2 of score s over the maximum (+inf over none, mu = -inf)
+__device__ __forceinline__ float over32(float s, float scale, const Max32& m) {
+  return __builtin_fmaf(s, scale, -m.mu) - m.res;
+}
+// Raise m to score s where that is larger; what was summed up scales by the result.
+__device__ __forceinline__ float raise32(Max32& m, float s, float scale) {
+  const bool up = over32(s, scale, m) > 0.f;
+  const Max32 n = max32_of(s, scale);
+  const float alpha = up ? fast_exp2((m.mu - n.mu) + (m.res - n.res)) : 1.f;
+  m.mu = up ? n.mu : m.mu;
+  m.res = up ? n.res : m.res;
+  return alpha;
+}
 
 // acc + x.lo + x.hi for a packed pair of 16-bit values (v_dot2 with (1, 1))
 template <bool BF>
@@ -946,15 +971,6 @@ __device__ __forceinline__ void st_dev4(float* p, f32x4 x) {
   st_dev2(p + 2, x2, x3);
 }
 
-// Weight of a partial with maximum m in a merge whose maximum is g.  The fp32
-// kernels keep m as a raw score and scale the difference: their scores may be
-// so large that the rounding of score * scale alone is worth many powers of two.
-template <int DT>
-__device__ __forceinline__ float part_weight(const KArgs& a, float m, float g) {
-  if constexpr (DT == FA2_DTYPE_F32) return fast_exp2((m - g) * a.ml_scale);
-  else return fast_exp2(m - g);
-}
-
 // Row r, columns col..col+3 of the unit in part slot `unit` (of S splits),
 // written to the output element offset `off`.
 template <int DT, int D>
@@ -988,13 +1004,13 @@ __device__ __forceinline__ void combine_row(const KArgs& a, int unit, int r, int
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // splits in order, as the one-at-a-time loop
-      const float wgt = part_weight<DT>(a, m[j], g_use);
+      const float wgt = fast_exp2(m[j] - g_use);
       lsum += wgt * l[j];
       acc += wgt * x[j];
     }
   }
   for (; s < S; ++s) {
-    const float wgt = part_weight<DT>(a, ml[s * ml_step], g_use);
+    const float wgt = fast_exp2(ml[s * ml_step] - g_use);
     lsum += wgt * ml[s * ml_step + 1];
     acc += wgt * *reinterpret_cast<const f32x4*>(po + s * o_step);
   }
@@ -1254,7 +1270,7 @@ __device__ __forceinline__ void merge_rows_sm(const KArgs& a, SlotOf slot_of, in
         for (int s = 0; s < SM; ++s) {
           if (s < S) {
             const uint32_t mw = ml[s][it][0], lw = ml[s][it][1];
-            const float wgt = part_weight<DT>(a, fl(mw), g_use);
+            const float wgt = fast_exp2(fl(mw) - g_use);
             lsum[it] += wgt * fl(lw);
             acc[it] += wgt * __builtin_bit_cast(f32x4, x[s][it]);
           }
@@ -1306,7 +1322,7 @@ __device__ __forceinline__ void merge_rows_sm(const KArgs& a, SlotOf slot_of, in
         for (int it = 0; it < kIt; ++it) {
           if (c0 + it * kRPP < rows) {
             const uint32_t mw = ml[it][0], lw = ml[it][1];
-            const float wgt = part_weight<DT>(a, fl(mw), g[it]);
+            const float wgt = fast_exp2(fl(mw) - g[it]);
             lsum[it] += wgt * fl(lw);
             acc[it] += wgt * __builtin_bit_cast(f32x4, x[it]);
           }

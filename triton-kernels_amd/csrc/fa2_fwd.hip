@@ -959,7 +959,6 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
   a.part_slots = static_cast<int32_t>(pl.grid_x);
   a.units = static_cast<int32_t>(pl.grid_pp);
   a.scale_log2 = p->softmax_scale * 1.4426950408889634f;
-  a.ml_scale = pl.f32 ? a.scale_log2 : 1.f;
   a.pool_bytes_k = pl.pool_bytes_k;
   a.pool_bytes_v = pl.pool_bytes_v;
   char* ws = static_cast<char*>(p->workspace);

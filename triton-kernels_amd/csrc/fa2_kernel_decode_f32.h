@@ -26,11 +26,8 @@
 //     K buffer, issued a phase earlier, gained 3 % on large two-block calls and
 //     spilled with one block at D = 128.)
 //   * The running max is raised, and O rescaled, only when a score passes it by
-//     2^8; the cross-lane maximum is skipped otherwise.  The max is kept as a raw
-//     score and the difference to it is scaled, (s - m) * scale, so that the largest
-//     weight is finite and not zero for scores of any finite size (an fma of s *
-//     scale against the rounded m * scale differs from it by the rounding of the
-//     product, 2^7 once that passes 2^31).
+//     2^8; the cross-lane maximum is skipped otherwise.  The largest weight is
+//     finite and not zero for scores of any finite size (Max32).
 //   * Rounding: with one block S is summed in eight chains and O in two levels
 //     (kFlush), so that the error against 64 bits stays at or below that of a
 //     tree over many lanes (2.1e-7 relative at 8192 keys).
@@ -94,8 +91,6 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
   const int seg_k = walk ? static_cast<int>(blockIdx.x) / a.walk_streams : 0;
 
   const float scale = a.scale_log2;
-  // kRescaleThreshold in units of a score (finite: the first maximum passes -inf)
-  const float rescale = fminf(kRescaleThreshold / scale, 3.4e38f);
 
   DecPiece p;
   DecSegment sg{};
@@ -204,7 +199,8 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
     // no key of a tile below this one is hidden from any row
     const int full = causal ? min(k_end, w.off + 1) : k_end;
 
-    float m[NB], l[NB];
+    Max32 m[NB];
+    float l[NB];
     f32x4 o[NB][DH][4];
     f32x4 o2[DH][4];  // kTwoLevel: the flushed sums
     float l2 = 0.f;
@@ -215,7 +211,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
       for (int e = 0; e < 4; ++e) o2[h][e] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      m[nb] = -INFINITY;
+      m[nb] = Max32{-INFINITY, 0.f};
       l[nb] = 0.f;
 #pragma unroll
       for (int h = 0; h < DH; ++h)
@@ -266,7 +262,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
           for (int r = 0; r < 4; ++r) s[nb][r] = n0 + 4 * g + r <= last[nb] ? s[nb][r] : -INFINITY;
         }
         mx[nb] = fmaxf(fmaxf(s[nb][0], s[nb][1]), fmaxf(s[nb][2], s[nb][3]));
-        need |= mx[nb] > m[nb] + rescale;
+        need |= over32(mx[nb], scale, m[nb]) > kRescaleThreshold;
       }
       if (__any(need)) {
 #pragma unroll
@@ -274,9 +270,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
           float x = mx[nb];
           x = fmaxf(x, __shfl_xor(x, 16));
           x = fmaxf(x, __shfl_xor(x, 32));
-          const float mn = fmaxf(m[nb], x);
-          const float alpha = fast_exp2((m[nb] - (mn == -INFINITY ? 0.f : mn)) * scale);
-          m[nb] = mn;
+          const float alpha = raise32(m[nb], x, scale);
           l[nb] *= alpha;
 #pragma unroll
           for (int h = 0; h < DH; ++h)
@@ -290,10 +284,10 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
       }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
-        const float mu = m[nb] == -INFINITY ? 0.f : m[nb];
+        const Max32 ref = m[nb].mu == -INFINITY ? Max32{0.f, 0.f} : m[nb];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[nb][r] = fast_exp2((s[nb][r] - mu) * scale);
+          s[nb][r] = fast_exp2(over32(s[nb][r], scale, ref));
           l[nb] += s[nb][r];
         }
       }
@@ -344,7 +338,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
       l[nb] += __shfl_xor(l[nb], 16);
       l[nb] += __shfl_xor(l[nb], 32);
       if (g == 0) {
-        mrg_ml[wave][nb * 16 + l16][0] = m[nb];
+        mrg_ml[wave][nb * 16 + l16][0] = m[nb].mu;
         mrg_ml[wave][nb * 16 + l16][1] = l[nb];
       }
     }
@@ -354,7 +348,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
       float mg = -INFINITY;
 #pragma unroll
       for (int x = 0; x < NW; ++x) mg = fmaxf(mg, mrg_ml[x][nb * 16 + l16][0]);
-      const float f = fast_exp2((m[nb] - (mg == -INFINITY ? 0.f : mg)) * scale);
+      const float f = fast_exp2(m[nb].mu - (mg == -INFINITY ? 0.f : mg));
       char* po = lds + wave * kOBytes + (nb * 16 + l16) * kOPitch + 16 * g * 4;
       if (nb * 16 + l16 < rows) {
 #pragma unroll
@@ -385,7 +379,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
         f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int x = 0; x < NW; ++x) {
-          lt += mrg_ml[x][r][1] * fast_exp2((mrg_ml[x][r][0] - mu) * scale);
+          lt += mrg_ml[x][r][1] * fast_exp2(mrg_ml[x][r][0] - mu);
           acc += *reinterpret_cast<const f32x4*>(lds + x * kOBytes + r * kOPitch + col * 4);
         }
         if (p.np == 1) {  // 0/0 -> NaN for a row with no key, as the reference

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_f32_kernel(
   f32x16 o[DB];
 #pragma unroll
   for (int d = 0; d < DB; ++d) o[d] = (f32x16){};
-  float m_run = -INFINITY;
+  Max32 m_run{-INFINITY, 0.f};
   float l_run = 0.f;
   const int wq_first = q0 + wave * kWaveRows;
   const int wq_diag = a.pack_m > 0 ? 0 : wq_first;
@@ -103,7 +103,6 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_f32_kernel(
   const int ksw = G::k(l32);
 
   const float scale = a.scale_log2;
-  const float rescale = fminf(kRescaleThreshold / scale, 3.4e38f);  // in units of a score
 
   if (T > 0) {
     ld.template issue<false>(a, w, t_begin * kBN, kbuf);
@@ -151,18 +150,15 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_f32_kernel(
 #pragma unroll
           for (int i2 = 0; i2 < 16; ++i2) mx = fmaxf(mx, s[sb][i2]);
         mx = max_xor32(mx);
-        // (the max is a raw score and the difference to it is scaled: finite
-        // weights for scores of any finite size, as in fa2_kernel_decode_f32.h)
-        const bool need = mx > m_run + rescale;
-        const float alpha = fast_exp2(need ? (m_run - mx) * scale : 0.0f);
-        m_run = need ? mx : m_run;
-        const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+        const bool need = over32(mx, scale, m_run) > kRescaleThreshold;
+        const float alpha = need ? raise32(m_run, mx, scale) : 1.0f;
+        const Max32 ref = m_run.mu == -INFINITY ? Max32{0.f, 0.f} : m_run;
         float rs = 0.f;
 #pragma unroll
         for (int sb = 0; sb < SB; ++sb)
 #pragma unroll
           for (int i2 = 0; i2 < 16; ++i2) {
-            s[sb][i2] = fast_exp2((s[sb][i2] - m_use) * scale);
+            s[sb][i2] = fast_exp2(over32(s[sb][i2], scale, ref));
             rs += s[sb][i2];
           }
         l_run = l_run * alpha + rs;
@@ -215,7 +211,7 @@ __global__ __launch_bounds__(kThreads, D > 128 ? 1 : 2) void fa2_fwd_f32_kernel(
     if (qrow < w.Lq && r < a.part_rows) {
       if (hi == 0) {
         float* ml = a.part_ml + (slot * a.part_rows + r) * 2;
-        ml[0] = m_run;
+        ml[0] = m_run.mu;
         ml[1] = l_tot;
       }
       float* po = a.part_o + (slot * a.part_rows + r) * D + hi * 4;
