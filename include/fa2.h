@@ -162,8 +162,9 @@ typedef struct fa2_params {
   /* fa2_decode_fwd, fp16/bf16: polls after which a wait of the
    * producer/consumer ring kernel gives up (0 = the library's bound, about
    * 5 ms; another value also selects that kernel, which otherwise serves
-   * forced splits and units of more than 16 rows).  A wait that gives up poisons its rows with NaN and counts in
-   * fa2_decode_wait_giveups().  Only tests set it, to exercise that path from
+   * forced splits, units of more than 16 rows, more than 65536 sequences and
+   * calls whose key tiles or partials leave 32-bit offsets).  A wait that
+   * gives up poisons its rows with NaN and counts in fa2_decode_wait_giveups().  Only tests set it, to exercise that path from
    * the host.  No counterpart in the reference, whose decode kernels do not
    * synchronise waves. */
   int32_t decode_spin_cap;
@@ -186,18 +187,24 @@ enum fa2_kernel {
   FA2_KERNEL_SHORT = 2
 };
 
-/* Bytes of device workspace fa2_fwd needs for `p` (0 is possible).
+/* Bytes of device workspace that suffice for fa2_fwd on `p` (0 is possible).
  * Replaces the reference's per-call torch.empty of running_sum/max/acc
- * (attention.py:852-864).  fp32 tensors with FA2_ARITH_REFERENCE at
- * head_dim 64/128 (dense, ragged) also hold fp16 copies of q, k and v and
- * one split's fp32 partials there, as the reference rounds every fp32 operand to
- * fp16 (also where the kernel that serves them needs only k and v).  Paged calls with one
+ * (attention.py:852-864).  For fp32 tensors with FA2_ARITH_REFERENCE at
+ * head_dim 64/128 (dense, ragged), which run on fp16 copies as the reference
+ * rounds every fp32 operand to fp16, this is the size of copies of q, k and v
+ * and one split's fp32 partials, whichever kernel serves the call;
+ * fa2_fwd_workspace_least tells what that kernel needs.  Paged calls with one
  * q-block per sequence and more two-head units than compute units hold the
  * partials of units their balanced walk cuts into pieces (4 * CUs * 128 *
  * (2 + head_dim) * 4 bytes).  Host-only: touches
  * no device state except a one-time, cached query of the current device's
  * compute-unit count. */
 int fa2_fwd_workspace_size(const fa2_params* p, size_t* bytes);
+
+/* The least workspace_bytes fa2_fwd accepts for `p`: at most
+ * fa2_fwd_workspace_size's, less where an fp32 call's kernel takes copies of k
+ * and v only, or writes its output itself.  Host-only, as above. */
+int fa2_fwd_workspace_least(const fa2_params* p, size_t* bytes);
 
 /* Validate `p` and enqueue the forward pass on `stream` (a hipStream_t;
  * NULL = the legacy default stream).  Replaces attention.py:836-925

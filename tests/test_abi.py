@@ -167,6 +167,40 @@ def test_fp32_workspace_holds_fp16_copies():
     assert (rc, n) == (0, 0)
 
 
+def rc_least(p):
+    n = ctypes.c_size_t(0)
+    return _fa2.lib().fa2_fwd_workspace_least(ctypes.byref(p), ctypes.byref(n)), n.value
+
+
+def test_fp32_least_workspace_follows_the_kernel():
+    """Copies of k and v for the one-head kernel (a grid that leaves CUs idle);
+    of q as well for the two-head kernel; partials where several splits or the
+    ragged two-head kernel write them.  fa2_fwd accepts exactly this much, and
+    it is no more than fa2_fwd_workspace_size, which other calls get."""
+    kv_el = 2 * 2 * 300 * 128
+    slack = 4096
+    small = dense_params(dtype=2)
+    rc, n = rc_least(small)
+    assert rc == 0 and 2 * 2 * kv_el <= n <= 2 * 2 * kv_el + slack
+    assert n < rc_ws(small)[1]
+    L, B, H, KH, D = 2048, 2, 32, 8, 128
+    big = dense_params(dtype=2, num_splits=0, q_heads=H, kv_heads=KH, q_len=L, kv_len=L)
+    big.q_sb, big.q_sh, big.q_ss = H * L * D, L * D, D
+    big.o_sb, big.o_sh, big.o_ss = big.q_sb, big.q_sh, big.q_ss
+    big.k_sb, big.k_sh, big.k_ss = KH * L * D, L * D, D
+    big.v_sb, big.v_sh, big.v_ss = big.k_sb, big.k_sh, big.k_ss
+    copies = 2 * B * L * D * (H + 2 * KH)
+    rc, n = rc_least(big)
+    assert rc == 0 and copies <= n <= copies + slack
+    rc, n = rc_least(dense_params(dtype=2, num_splits=4))
+    assert rc == 0 and n >= 4 * (3 * 2 * 8) * 128 * (2 + 128) * 4 + 4 * kv_el
+    for p in (small, big, dense_params(dtype=2, num_splits=4)):
+        p.q = p.k = p.v = p.o = p.workspace = 16
+        p.workspace_bytes = rc_least(p)[1] - 1
+        assert rc_fwd(p) == 10
+    assert rc_least(dense_params(num_splits=4)) == rc_ws(dense_params(num_splits=4))
+
+
 def test_workspace_too_small_is_rejected():
     p = dense_params(num_splits=2, q=16, k=16, v=16, o=16)
     rc, n = rc_ws(p)

@@ -118,6 +118,17 @@ def test_noalloc_reduces_splits_to_fit():
     check_all(case, "dense", False, unpack(case, "dense", out, kw))
 
 
+def test_noalloc_fp32_takes_what_its_kernel_needs():
+    """2 x 1500 rows of fp32, Hq16/Hkv4 D128: copies of k and v (6 MB) fit the
+    scratch, those of q and partials, which this kernel does not use, would
+    not: the call runs fa2_fwd's kernel, bit for bit."""
+    case = make_case(2, 16, 4, 128, "self", torch.float32, "dense", 6300,
+                     dense_q_range=(1500, 1500))
+    q, k, v, kw = pack(case, "dense", device=DEV)
+    assert torch.equal(call(q, k, v, kw, True, "dense", True).view(torch.int32),
+                       call(q, k, v, kw, True, "dense", False).view(torch.int32))
+
+
 def test_noalloc_paged_runs_whole_units():
     """40 paged sequences of one q-block over 128-1800 keys, Hq16/Hkv4: 320
     two-head units, more than the CUs, so fa2_fwd takes the balanced walk

@@ -165,6 +165,7 @@ struct Plan {
   int64_t max_wgs;  // cap on the persistent grid (0: none)
   uint32_t pool_bytes_k, pool_bytes_v;
   size_t off_work, off_count, off_ml, off_o, off_ctr, off_cq, off_ck, off_cv, total;
+  size_t told;      // the size callers are told: total, or more (finish_plan)
 };
 
 // K/V tiles are read through buffer descriptors.  Dense and ragged tiles, and
@@ -511,19 +512,18 @@ int finish_plan(const fa2_params* p, Plan* pl) {
   else if (pl->fold || pl->bal)
     off += static_cast<size_t>(pl->grid_x) * sizeof(uint64_t);
   off = (off + 255) & ~size_t(255);
-  const size_t slots = pl->walk  ? static_cast<size_t>(2 * pl->walk_streams * pl->walk_segs)  // two cut pieces per workgroup
+  // (walk: two cut pieces per workgroup of a segment)
+  const size_t slots = pl->walk  ? static_cast<size_t>(2 * pl->walk_streams * pl->walk_segs)
                        : pl->bal ? static_cast<size_t>(pl->bal_slots)
-                       : parts || pl->conv ? static_cast<size_t>(splits) * pl->grid_x
+                       : parts   ? static_cast<size_t>(splits) * pl->grid_x
                                  : 0;
   pl->off_ml = off;
   off += slots * pl->part_rows * 2 * sizeof(float);
   off = (off + 255) & ~size_t(255);
   pl->off_o = off;
   off += slots * pl->part_rows * pl->dim * sizeof(float);
-  // fp16 copies: q [B][Hq][Lq][D] or [Tq][Hq][D], k and v likewise.  (The size
-  // told to callers holds q's copy and one split's partials for every such call,
-  // also where its kernel needs neither, so that it does not hang on which
-  // kernel serves the call.)
+  // fp16 copies: k and v [B][Hkv][N][D] or [Tkv][Hkv][D], and for the two-head
+  // kernel q likewise
   const int64_t qrows = p->layout == FA2_LAYOUT_DENSE ? p->batch * p->q_len : p->q_len;
   const int64_t kvrows = p->layout == FA2_LAYOUT_DENSE ? p->batch * p->kv_len : p->kv_len;
   auto copy = [&](size_t& at, int64_t rows, int64_t heads) {
@@ -531,10 +531,16 @@ int finish_plan(const fa2_params* p, Plan* pl) {
     at = off;
     if (pl->conv) off += static_cast<size_t>(rows) * heads * p->head_dim * 2;
   };
-  copy(pl->off_cq, qrows, p->q_heads);
+  copy(pl->off_cq, pl->pp ? qrows : 0, p->q_heads);
   copy(pl->off_ck, kvrows, p->kv_heads);
   copy(pl->off_cv, kvrows, p->kv_heads);
-  pl->total = off;
+  pl->total = pl->told = off;
+  if (pl->conv) {  // also what the other kernel would take: q's copy, one split's partials
+    if (!pl->pp) pl->told += static_cast<size_t>(qrows) * p->q_heads * p->head_dim * 2 + 256;
+    if (!parts)
+      pl->told += static_cast<size_t>(splits) * pl->grid_x * pl->part_rows * (2 + pl->dim) *
+                      sizeof(float) + 512;
+  }
   return FA2_OK;
 }
 
@@ -878,7 +884,7 @@ extern "C" const char* fa2_strerror(int s) {
 namespace fa2 {
 namespace {
 
-int workspace_size(const fa2_params* p, size_t* bytes, bool packed) {
+int workspace_size(const fa2_params* p, size_t* bytes, bool packed, bool least = false) {
   if (!bytes) return FA2_ERR_NULL_POINTER;
   int s = packed ? validate_decode(p) : validate(p);
   if (s != FA2_OK) return s;
@@ -890,7 +896,7 @@ int workspace_size(const fa2_params* p, size_t* bytes, bool packed) {
   s = packed ? make_plan_packed(p, &pl, p->num_splits == 0)
              : make_plan(p, &pl, p->num_splits == 0);
   if (s != FA2_OK) return s;
-  *bytes = pl.total;
+  *bytes = least ? pl.total : pl.told;
   return FA2_OK;
 }
 
@@ -1061,6 +1067,10 @@ int run(const fa2_params* p, void* stream, bool packed, bool allow_conv = true,
 
 extern "C" int fa2_fwd_workspace_size(const fa2_params* p, size_t* bytes) {
   return workspace_size(p, bytes, false);
+}
+
+extern "C" int fa2_fwd_workspace_least(const fa2_params* p, size_t* bytes) {
+  return workspace_size(p, bytes, false, true);
 }
 
 extern "C" int fa2_fwd(const fa2_params* p, void* stream) { return run(p, stream, false); }

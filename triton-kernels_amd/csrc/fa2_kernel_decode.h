@@ -1,7 +1,8 @@
 // fa2_kernel_decode.h - fp16/bf16 kernel of decode_attention and
 // speculative_decode_attention (packed-head mode, KArgs::pack_m > 0) for forced
-// split counts, a lowered spin cap, units of more than 16 rows and more than
-// 4096 sequences; fa2_kernel_decode_wave.h serves the others.
+// split counts, a lowered spin cap, units of more than 16 rows, more than 65536
+// sequences, and calls whose key tiles or partials leave 32-bit offsets;
+// fa2_kernel_decode_wave.h serves the others.
 //
 // These calls read every K/V row once per kv head and do little arithmetic
 // per byte (4 * rows FLOP per K/V element, rows = Hq/Hkv * M <= 64 per

@@ -141,7 +141,7 @@ at::Tensor fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout, int64_t
   }
 
   size_t ws_bytes = 0;
-  int rc = fa2_fwd_workspace_size(&p, &ws_bytes);
+  int rc = fa2_fwd_workspace_least(&p, &ws_bytes);
   TORCH_CHECK(rc == FA2_OK, "flash_attention_v2: ", fa2_strerror(rc), " (fa2 status ", rc, ")");
   at::Tensor ws;
   if (ws_bytes) {

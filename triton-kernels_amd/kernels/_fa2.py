@@ -26,7 +26,7 @@ MAX_SPLITS = 64
 ABI_VERSION = 7
 
 # Every symbol include/fa2.h declares.
-EXPORTS = ("fa2_fwd_workspace_size", "fa2_fwd", "fa2_fwd_noalloc", "fa2_strerror",
+EXPORTS = ("fa2_fwd_workspace_size", "fa2_fwd_workspace_least", "fa2_fwd", "fa2_fwd_noalloc", "fa2_strerror",
            "fa2_decode_workspace_size", "fa2_decode_fwd", "fa2_decode_wait_giveups",
            "fa2_kv_append",
            "fa2_kv_append_params_size", "fa2_abi_version", "fa2_params_size")
@@ -105,6 +105,9 @@ def lib():
             L.fa2_fwd_workspace_size.argtypes = [ctypes.POINTER(Fa2Params),
                                                  ctypes.POINTER(ctypes.c_size_t)]
             L.fa2_fwd_workspace_size.restype = ctypes.c_int
+            L.fa2_fwd_workspace_least.argtypes = [ctypes.POINTER(Fa2Params),
+                                                  ctypes.POINTER(ctypes.c_size_t)]
+            L.fa2_fwd_workspace_least.restype = ctypes.c_int
             L.fa2_fwd.argtypes = [ctypes.POINTER(Fa2Params), ctypes.c_void_p]
             L.fa2_fwd.restype = ctypes.c_int
             L.fa2_fwd_noalloc.argtypes = [ctypes.POINTER(Fa2Params), ctypes.c_void_p]
@@ -144,9 +147,9 @@ class Fa2Error(RuntimeError):
 
 
 def workspace_size(p: Fa2Params, decode: bool = False) -> int:
-    """Device workspace bytes of ``fa2_fwd`` (or ``fa2_decode_fwd``) for ``p``."""
+    """Device workspace bytes ``fa2_fwd`` (or ``fa2_decode_fwd``) takes for ``p``."""
     n = ctypes.c_size_t(0)
-    fn = lib().fa2_decode_workspace_size if decode else lib().fa2_fwd_workspace_size
+    fn = lib().fa2_decode_workspace_size if decode else lib().fa2_fwd_workspace_least
     rc = fn(ctypes.byref(p), ctypes.byref(n))
     if rc != 0:
         raise Fa2Error(rc)
