@@ -432,13 +432,15 @@ int make_plan(const fa2_params* p, Plan* pl, bool query_device, bool allow_conv 
   // neither the plan nor the combine kernel is launched.
   //   Workgroups of further automatic splits need not be resident with the
   // first (the last split to finish merges, none waits) where the lengths will
-  // most likely cancel them: a mean of fewer tiles than two splits take, and at
-  // most 4 of them.  Measured on MI355X, plan + combine against none: 16
-  // sequences of 17-128 rows over 65-511 keys, Hq8/Hkv2 D128, three splits by
-  // the host's bound, one by the lengths, 23.3 -> 18.7 us (plan 4, combine 4).
-  // Where the splits run, the merge by one workgroup takes longer than the
-  // combine kernel's grid: 17 x 4096 keys, 4 splits, 72 -> 74 us; 3 x 8000 keys
-  // Hq32/Hkv8, 6 splits, 78 -> 84; 8 x 4096, 8 forced, 41 -> 63.
+  // most likely cancel them: a mean below the tiles of one split, of which lengths
+  // spread from none to twice the mean leave one, and at most 4 by the host's bound.
+  // Measured on MI355X, plan + combine against none: 16 sequences of 17-128 rows
+  // over 65-511 keys, Hq8/Hkv2 D128, three splits by the host's bound, one by the
+  // lengths, 23.3 -> 18.7 us (plan 4, combine 4).  Where the splits run, the merge
+  // by one workgroup takes longer than the combine kernel's grid: 11 x 1500 keys
+  // and one of 6000, Hq8/Hkv2, 70 -> 76; 15 x 300 and one of 20000, Hq16/Hkv4, 217
+  // -> 229 (means of 1875 and 1531); 31 x 300 and one of 20000, which the mean of
+  // 916 lets through, 216 -> 228.
   pl->inline_plan = false;
   const bool lds_dim = p->head_dim == 64 || p->head_dim == 128 || p->head_dim == 256;
   if (FA2_INLINE_PLAN && p->layout == FA2_LAYOUT_RAGGED && half && !pl->conv && !pl->f32 &&
@@ -447,7 +449,7 @@ int make_plan(const fa2_params* p, Plan* pl, bool query_device, bool allow_conv 
     const int64_t resident = pl->pp ? 1 : (p->head_dim > 128 ? 1 : FA2_LDS_OCCUPANCY);
     const int64_t per_split = pl->pp ? pl->grid_pp : pl->grid_x;
     const bool cancelled = p->num_splits == 0 && splits <= 4 &&
-                           kv_upper_bound(p) < int64_t(p->batch) * 2 * kMinSplitTiles * kBN;
+                           kv_upper_bound(p) < int64_t(p->batch) * kMinSplitTiles * kBN;
     if (per_split * (cancelled ? 1 : splits) <= cus * resident) {
       pl->inline_plan = true;
       pl->plan = false;
