@@ -155,12 +155,14 @@ def test_forced_splits(layout, splits):
     check(case, layout, run(case, layout, num_splits=splits))
 
 
+@pytest.mark.parametrize("heads", [(4, 2), (34, 2)], ids=["walk", "plan"])
 @pytest.mark.parametrize("B", [255, 256, 257, 700])
 @pytest.mark.parametrize("layout", ["ragged", "paged"])
-def test_batch_sizes_around_the_plan_fast_path(layout, B):
-    """The device plan ranks up to 256 sequences directly and counting-sorts
-    larger batches: either order must cover every sequence exactly once."""
-    case = make_decode_case(B, 4, 2, 64, 1, torch.bfloat16, layout, seed=3600 + B,
+def test_batch_sizes_around_the_plan_fast_path(layout, B, heads):
+    """The device plan of units of more than 16 rows ranks up to 256 sequences
+    directly and counting-sorts larger batches; smaller units walk them, several
+    sequences per lane.  Either order must cover every sequence exactly once."""
+    case = make_decode_case(B, *heads, 64, 1, torch.bfloat16, layout, seed=3600 + B,
                             kv_range=(1, 80))
     check(case, layout, run(case, layout, decode=True))
 
@@ -272,10 +274,11 @@ def test_assertions_match_reference():
                          torch.randn((2, 3, 10, 64), device=DEV, dtype=torch.float16))
 
 
+@pytest.mark.parametrize("splits", [0, 5], ids=["walk", "splits"])
 @pytest.mark.parametrize("fill", ["zeros", "ones", "random", "reused"])
-def test_split_merge_words_need_no_clearing(fill):
-    """A split decode call merges its splits inside the kernel: the last
-    split of a unit to finish combines the partials, counted in one 64-bit
+def test_split_merge_words_need_no_clearing(fill, splits):
+    """A decode call merges its splits, or the pieces of a unit the walk cuts,
+    inside the kernel: the last of a unit to finish combines the partials, counted in one 64-bit
     word per unit of the workspace that holds a per-call tag.  Whatever the
     workspace held before (never cleared: zeros, all ones, random bytes, the
     words a previous call left), the output must equal that of a call on a
@@ -283,7 +286,7 @@ def test_split_merge_words_need_no_clearing(fill):
     from kernels import _fa2
     from kernels.decode import _run_decode
     g = torch.Generator(device=DEV).manual_seed(4242)
-    B, QH, KVH, D, N = 4, 16, 2, 128, 3000  # 8 units of 47 tiles: 5 automatic splits
+    B, QH, KVH, D, N = 4, 16, 2, 128, 3000  # 8 units of 47 tiles
     q = torch.randn(B, QH, D, generator=g, device=DEV).to(torch.bfloat16)
     k = torch.randn(B, KVH, N, D, generator=g, device=DEV).to(torch.bfloat16)
     v = torch.randn(B, KVH, N, D, generator=g, device=DEV).to(torch.bfloat16)
@@ -294,7 +297,7 @@ def test_split_merge_words_need_no_clearing(fill):
         _run_decode("decode_attention", q.unsqueeze(2), k, v, out.unsqueeze(2),
                     layout=_fa2.LAYOUT_DENSE, causal=False, batch=B, q_heads=QH, kv_heads=KVH,
                     head_dim=D, kv_indptr=None, k_block_table=None, v_block_table=None,
-                    kv_page_size=None, workspace=ws)
+                    kv_page_size=None, num_splits=splits, workspace=ws)
         torch.cuda.synchronize()
         return out
 

@@ -13,7 +13,7 @@ different maxima), so they agree within the strict bar's own floor.
 import pytest
 import torch
 
-from decode_cases import LAYOUTS, make_decode_case
+from decode_cases import LAYOUTS, make_decode_case, pack_decode
 from test_decode_gpu import check, run
 
 pytestmark = pytest.mark.gpu
@@ -145,3 +145,67 @@ def test_many_units_f32(layout, D, heads, M, splits):
     case = make_decode_case(B, QH, KVH, D, M, torch.float32, layout, seed=5850 + M, causal=M > 1,
                             ctx_lens=lens)
     check(case, layout, run(case, layout, num_splits=splits))
+
+
+# ---- more sequences than lanes: several per lane of the locating wave ----
+
+@pytest.mark.parametrize("B", [65, 129, 700])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("layout", ["ragged", "paged"])
+def test_cut_units_among_many_sequences(layout, dt, B):
+    """Mostly short and empty sequences and a few of 47 tiles, which are cut: the
+    starts of the segments lie inside the lanes' groups of sequences."""
+    lens = [7 * i % 40 for i in range(B)]
+    for i in (0, 3, B // 2, B - 2):
+        lens[i] = 3000 + i % 64
+    case = make_decode_case(B, 4, 2, 64, 1, dt, layout, seed=5900 + B, ctx_lens=lens)
+    check(case, layout, run(case, layout, decode=True))
+
+
+@pytest.mark.parametrize("B", [4096, 4097])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_cut_units_among_thousands_of_sequences(dt, B):
+    lens = [i % 3 for i in range(B)]
+    lens[B // 2] = 3000
+    case = make_decode_case(B, 2, 2, 64, 1, dt, "ragged", seed=5950 + B, ctx_lens=lens)
+    check(case, "ragged", run(case, "ragged", decode=True))
+
+
+@pytest.mark.parametrize("B", [65536, 65537])
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32], ids=["fp16", "fp32"])
+def test_sequences_at_the_walks_limit(dt, B):
+    """One past it the other decode kernels run, with a plan by list (dense: none)."""
+    from kernels import decode_attention
+    g = torch.Generator().manual_seed(B)
+    q, k, v = (torch.randn(s, generator=g).to(dt) for s in ((B, 2, 64), (B, 1, 3, 64), (B, 1, 3, 64)))
+    out = decode_attention(q.cuda(), k.cuda(), v.cuda()).cpu().double()
+    s = torch.matmul(q.double(), k[:, 0].double().transpose(1, 2).contiguous()) / 8
+    ref = torch.matmul(torch.softmax(s, -1), v[:, 0].double())
+    # fp16: weights and output rounded to 11 bits, |v| < 6; fp32: a few ulps of it
+    assert (out - ref).abs().max().item() < (6 * 2.0 ** -9 if dt == torch.float16 else 1e-5)
+
+
+# ---- strides: heads outside the rows ----
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("M", [1, 3])
+def test_strided_caches_equal_contiguous_ones(layout, D, dt, M):
+    """Head-major pools and token rows, dense K and V as views of [B, N, H, D], a K
+    whose rows lie further apart than V's: no copy is made, the same bits."""
+    from kernels import speculative_decode_attention
+    lens = [1100] * 3 if layout == "dense" else LENS
+    case = make_decode_case(len(lens), 8, 4, D, M, dt, layout, seed=5980 + M, causal=M > 1,
+                            ctx_lens=lens)
+    pk = dict(shuffled=True, page=16) if layout == "paged" else {}
+    q, k, v, kw = pack_decode(case, layout, device="cuda", **pk)
+    a = speculative_decode_attention(q, k, v, causal=M > 1, **kw)
+    i, j = (1, 2) if layout == "dense" else (0, 1)
+    ks, vs = (t.transpose(i, j).contiguous().transpose(i, j) for t in (k, v))
+    wide = torch.full((*k.shape[:-1], 3 * D), float("nan"), dtype=dt, device="cuda")
+    wide[..., D:2 * D] = k
+    for kk, vv in ((ks, vs), (ks, v), (wide[..., D:2 * D], vs)):
+        b = speculative_decode_attention(q, kk, vv, causal=M > 1, **kw)
+        # (an empty sequence's rows are NaN in both)
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0), b.nan_to_num(0))

@@ -91,13 +91,20 @@ def test_paged_pool_over_2gib(qh, kvh, dtype, kernel, page, causal):
     torch.cuda.empty_cache()
 
 
+# (drafts, forced splits): 16 rows per unit, the wave-streaming kernel; 48 rows and
+# forced splits, the ring kernel.  fp32: the fp32 decode kernel, one and two blocks.
+DECODES = [(4, 0), (12, 0), (4, 3)]
+DECODE_IDS = ["rows16", "rows48", "splits"]
+
+
+@pytest.mark.parametrize("M,splits", DECODES, ids=DECODE_IDS)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
 @pytest.mark.parametrize("page", [16, 5])
-def test_decode_pool_over_2gib(dtype, page):
-    """speculative_decode_attention (the decode kernel; fp32: the
-    register-staged kernel in packed mode) over a pool past 2 GiB."""
+def test_decode_pool_over_2gib(dtype, page, M, splits):
+    """speculative_decode_attention over a pool past 2 GiB (the ring kernel's
+    BUF = false instantiation)."""
     from kernels import speculative_decode_attention
-    case = make_decode_case(3, 8, 2, 128, 4, dtype, "paged", 5100 + page, causal=True,
+    case = make_decode_case(3, 8, 2, 128, M, dtype, "paged", 5100 + page, causal=True,
                             kv_range=(100, 900))
     kc, kt = big_pool(case.ks, page, GIB2 + (64 << 20), 3)
     vc, vt = big_pool(case.vs, page, GIB2 + (64 << 20), 4)
@@ -105,7 +112,7 @@ def test_decode_pool_over_2gib(dtype, page):
     out = speculative_decode_attention(
         q, kc, vc, causal=True, kv_indptr=torch.tensor(case.kv_lens, dtype=torch.int32,
                                                        device=DEV),
-        k_block_table=kt, v_block_table=vt, kv_page_size=page)
+        k_block_table=kt, v_block_table=vt, kv_page_size=page, num_splits=splits)
     torch.cuda.synchronize()
     out = out.cpu()
     check_decode(case, "paged", [out[b] for b in range(3)])
@@ -190,22 +197,24 @@ def test_paged_unknown_pool_size(qh, kvh, dtype, kernel, page, causal, splits):
     check_all(case, "paged", causal, unpack(case, "paged", out.cpu(), kw))
 
 
+@pytest.mark.parametrize("QH,splits", [(8, 0), (40, 0), (8, 3)], ids=["rows4", "rows20", "splits"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
 @pytest.mark.parametrize("page", [16, 5])
-def test_decode_unknown_pool_size(dtype, page):
-    """decode with kv_len = 0 through the ABI (the decode kernel's BUF = false
-    instantiation), bitwise against the call with the pool size."""
+def test_decode_unknown_pool_size(dtype, page, QH, splits):
+    """decode with kv_len = 0 through the ABI (rows clamped to no pool; more than 16
+    rows or forced splits: the ring kernel's BUF = false instantiation), bitwise
+    against the call with the pool size."""
     from kernels import _fa2, decode_attention
     from kernels._launch import enqueue, index_tensor, table
-    case = make_decode_case(4, 8, 2, 128, 1, dtype, "paged", 5400 + page, kv_range=(1, 900))
+    case = make_decode_case(4, QH, 2, 128, 1, dtype, "paged", 5400 + page, kv_range=(1, 900))
     q, k, v, kw = pack_decode(case, "paged", device=DEV, shuffled=True, seed=page, page=page,
                               squeeze_m=True)
-    ref = decode_attention(q, k, v, **kw)
+    ref = decode_attention(q, k, v, num_splits=splits, **kw)
     out = torch.empty_like(q)
     q4, o4 = q.unsqueeze(2), out.unsqueeze(2)
     ab = lambda t: (t.stride(0), t.stride(1), t.stride(1))  # noqa: E731 (M = 1)
-    enqueue(decode=True, layout=_fa2.LAYOUT_PAGED, mask=_fa2.MASK_NONE, num_splits=0,
-            batch=4, q_heads=8, kv_heads=2, head_dim=128, q_len=1, kv_len=0, q=q4, k=k, v=v,
+    enqueue(decode=True, layout=_fa2.LAYOUT_PAGED, mask=_fa2.MASK_NONE, num_splits=splits,
+            batch=4, q_heads=QH, kv_heads=2, head_dim=128, q_len=1, kv_len=0, q=q4, k=k, v=v,
             out=o4, q_strides=ab(q4), o_strides=ab(o4),
             kvi=index_tensor(kw["kv_indptr"], q.device), kt=table(kw["k_block_table"], q.device),
             vt=table(kw["v_block_table"], q.device), page_size=page,
