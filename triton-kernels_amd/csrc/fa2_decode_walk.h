@@ -95,9 +95,9 @@ struct DecSegment {
 };
 
 // Whether units of up to `longest` tiles stay whole, walk_rounds of them per
-// workgroup, rather than C tiles of cut ones.
-__device__ __forceinline__ bool walk_keep_whole(const KArgs& a, int longest, int C) {
-  return longest <= a.walk_short || a.walk_rounds <= (C + a.walk_whole) / longest;
+// workgroup, rather than C tiles of cut ones; `cost`: tiles' time of cutting them.
+__device__ __forceinline__ bool walk_keep_whole(const KArgs& a, int longest, int C, int cost) {
+  return longest <= a.walk_short || a.walk_rounds <= (C + cost) / longest;
 }
 
 // By one wave: segment k of a stream into *sh (LDS); k >= walk_segs: empty.
@@ -110,7 +110,8 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
       const int W = walk_weight<TK>(a.kv_len);
       const int total = W * a.batch;
       const int C = max((total + segs - 1) / segs, a.walk_min);
-      if (walk_keep_whole(a, W, C)) {
+      // (shares that no two units lie in have one piece to merge, not two)
+      if (walk_keep_whole(a, W, C, W % C == 0 ? a.walk_whole / 2 : a.walk_whole)) {
         *sh = DecSegment{k, 0, 0, 0, 0};
         return;
       }
@@ -140,7 +141,7 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
   }
   const int total = __shfl(incl, 63);
   const int C = max((total + segs - 1) / segs, a.walk_min);
-  if (walk_keep_whole(a, longest, C)) {
+  if (walk_keep_whole(a, longest, C, a.walk_whole)) {
     if (lane == 0) *sh = DecSegment{k, 0, 0, 0, 0};
     return;
   }

@@ -87,13 +87,18 @@ constexpr int64_t kDecMinTiles = 4;
 // tiles of the call per workgroup of the walks at least
 constexpr int64_t kWalkGridTiles = 2;
 // Whole units of the walks (KArgs::walk_whole, walk_short), in KV tiles of 64 keys.
-// Measured on MI355X, kernel time in us, cut / whole.  16 bits, D64: 4 x 500-1500
-// keys Hkv8 25 / 10, 16 x 500-1500 Hkv8 22 / 15.5, 16 x 2048 Hkv1 15 / 12, 64 x
-// 2000-6000 Hkv8 111 / 119.  D128: 4 x 500-1500 Hkv8 21 / 15, 16 x 500-1500
-// Hkv8 21.6 / 23.5, 16 x 2048 Hkv4 18 / 24, 1 x 2048 Hkv96 24 / 29, 300 x 600-768
-// Hkv1 30 / 27.  fp32, D128: 1 x 500 Hkv4 12.7 / 18, 4 x 500 Hkv8 14 / 18, 33 x
-// 330-384 Hkv8 34 / 38.
-constexpr int64_t kWholeIdle = 24, kWholeBusy = 12, kWholeShort = 12;
+// In 16 bits cutting costs the time of up to kWholeIdle tiles, in proportion to the
+// CUs that the call's units leave idle (where a tile is mostly latency), and of
+// kWholeBusy at least; twice as many and more at head_dim 64, whose tiles are half
+// the bytes.  Measured on MI355X, kernel time in us, cut / whole.  D64: 4 x
+// 500-1500 keys Hkv8 25 / 10, 16 x 500-1500 Hkv8 22 / 15.5, 4 x 3000 Hkv8 22 / 16, 1
+// x 3000 Hkv4 10 / 15, 64 x 2000-6000 Hkv8 111 / 119.  D128: 4 x 500-1500 Hkv8 21
+// / 15, 4 x 1023 Hkv8 12.7 / 14.2, 16 x 500-1500 Hkv8 21.6 / 23.5, 16 x 2048 Hkv4
+// 18 / 24, 1 x 2048 Hkv96 24 / 29, 300 x 600-768 Hkv1 30 / 27.  fp32, D128: 1 x 500
+// Hkv4 12.7 / 18, 4 x 500 Hkv8 14 / 18, 33 x 330-384 Hkv8 34 / 38.
+constexpr int64_t kWholeIdle128 = 20, kWholeIdle64 = 48;
+constexpr int64_t kWholeBusy128 = 12, kWholeBusy64 = 24;
+constexpr int64_t kWholeShort = 12;
 constexpr int64_t kWholeF32 = 2, kWholeShortF32 = 4;
 
 // byte offset of the kXcds claim counters after the work list's item count
@@ -663,14 +668,12 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
       // fp32: more workgroups, which only take whole units
       if (pl->decf32) pl->grid_x = std::max(pl->grid_x, std::min(wgs, streams * p->batch));
       if (wave) pl->block_rows = kDwRows;
-      // What cutting costs in 16 bits, in tiles: more where few units leave most
-      // CUs idle and a tile is mostly latency, twice as many at head_dim 64, whose
-      // tiles are half the bytes.
       const int64_t idle = std::max<int64_t>(0, pl->grid_x - streams * p->batch);
-      pl->walk_whole = pl->decf32 ? kWholeF32
-                                  : std::max(kWholeBusy * 128 / pl->dim,
-                                             (pl->dim == 64 ? 3 : 2) * kWholeIdle * idle /
-                                                 (2 * pl->grid_x));
+      const bool d64 = pl->dim == 64;
+      pl->walk_whole = pl->decf32
+                           ? kWholeF32
+                           : std::max(d64 ? kWholeBusy64 : kWholeBusy128,
+                                      (d64 ? kWholeIdle64 : kWholeIdle128) * idle / pl->grid_x);
       pl->walk_short = pl->decf32 ? kWholeShortF32 : kWholeShort;
     }
   }
