@@ -164,7 +164,8 @@ typedef struct fa2_params {
    * 5 ms; another value also selects that kernel, which otherwise serves
    * forced splits, units of more than 16 rows, more than 65536 sequences and
    * calls whose key tiles or partials leave 32-bit offsets).  A wait that
-   * gives up poisons its rows with NaN and counts in fa2_decode_wait_giveups().  Only tests set it, to exercise that path from
+   * gives up poisons its rows with NaN and counts in
+   * fa2_decode_wait_giveups().  Only tests set it, to exercise that path from
    * the host.  No counterpart in the reference, whose decode kernels do not
    * synchronise waves. */
   int32_t decode_spin_cap;

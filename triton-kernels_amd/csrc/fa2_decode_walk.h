@@ -3,8 +3,8 @@
 //
 // A call's units are (sequence, kv head, q-block).  The kv heads and
 // q-blocks form a.walk_streams streams; stream s holds the units (b, s) of
-// all sequences in order, unit b weighing max(1, ceil(Lk_b / TK)) tiles of
-// TK = 64 keys.  The grid starts with walk_streams * walk_segs workgroups:
+// all sequences in order, unit b weighing max(1, ceil(Lk_b / kBN)) tiles
+// of kBN = 64 keys.  The grid starts with walk_streams * walk_segs workgroups:
 // workgroup g takes stream g % walk_streams and segment k = g / walk_streams of
 // it, tiles [k C, (k + 1) C) with C = ceil(total / walk_segs), at least
 // a.walk_min.  The kv heads of a sequence are therefore read at about the same
@@ -49,9 +49,8 @@ __device__ __forceinline__ int walk_len(const KArgs& a, int b) {
   return n > 0 ? n : 0;
 }
 
-template <int TK>
 __device__ __forceinline__ int walk_weight(int Lk) {
-  const int t = (Lk + TK - 1) / TK;
+  const int t = (Lk + kBN - 1) / kBN;
   return t > 1 ? t : 1;
 }
 
@@ -101,13 +100,13 @@ __device__ __forceinline__ bool walk_keep_whole(const KArgs& a, int longest, int
 }
 
 // By one wave: segment k of a stream into *sh (LDS); k >= walk_segs: empty.
-template <int MODE, int TK>
+template <int MODE>
 __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* sh) {
   const int lane = threadIdx.x & 63;
   const int segs = a.walk_segs;
   if constexpr (MODE == FA2_LAYOUT_DENSE) {
     if (lane == 0) {
-      const int W = walk_weight<TK>(a.kv_len);
+      const int W = walk_weight(a.kv_len);
       const int total = W * a.batch;
       const int C = max((total + segs - 1) / segs, a.walk_min);
       // (shares that no two units lie in have one piece to merge, not two)
@@ -124,7 +123,7 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
   const int j0 = min(a.batch, lane * per), j1 = min(a.batch, j0 + per);
   int sum = 0, longest = 0;
   for (int j = j0; j < j1; ++j) {
-    const int W = walk_weight<TK>(walk_len<MODE>(a, j));
+    const int W = walk_weight(walk_len<MODE>(a, j));
     sum += W;
     longest = max(longest, W);
   }
@@ -150,7 +149,7 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
   if (excl <= s0 && s0 < incl) {  // one lane, or none past the end
     int us = excl, j = j0;
     for (;; ++j) {
-      const int W = walk_weight<TK>(walk_len<MODE>(a, j));
+      const int W = walk_weight(walk_len<MODE>(a, j));
       if (s0 < us + W) break;
       us += W;
     }
@@ -162,13 +161,13 @@ __device__ __forceinline__ void walk_locate(const KArgs& a, int k, DecSegment* s
 
 // The piece of sequence j's unit (starting at us in its stream) that falls
 // in segment g (whole units: all of it); false past the segment's end.
-template <int MODE, int TK>
+template <int MODE>
 __device__ __forceinline__ bool walk_piece(const KArgs& a, const DecSegment& g, int stream, int k,
                                            int j, int us, DecPiece& p) {
   const bool whole = g.C == 0;
   if (j >= a.batch || (!whole && us >= g.s1)) return false;
   p.w = packed_work<MODE>(a, j, stream % a.hkv, stream / a.hkv);
-  const int tiles = (p.w.Lk + TK - 1) / TK;
+  const int tiles = (p.w.Lk + kBN - 1) / kBN;
   p.us = us;
   p.W = tiles > 1 ? tiles : 1;
   p.unit = j * a.walk_streams + stream;
@@ -210,11 +209,11 @@ __device__ __forceinline__ void walk_next_unit(const KArgs& a, const DecSegment&
 }
 
 // Split blockIdx.y of unit blockIdx.x (no walk); false: no such unit.
-template <int MODE, int TK>
+template <int MODE>
 __device__ __forceinline__ bool split_piece(const KArgs& a, DecPiece& p) {
   p.w = decode_work<MODE>(a, blockIdx.x);
   if (!p.w.valid) return false;
-  const int tiles = (p.w.Lk + TK - 1) / TK;
+  const int tiles = (p.w.Lk + kBN - 1) / kBN;
   // (splits past the unit's tiles would have none: they are not counted)
   const int S = a.merge_ctr ? min(a.num_splits, max(tiles, 1)) : a.num_splits;
   const int split = blockIdx.y;

@@ -621,9 +621,9 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   pl->part_rows = static_cast<int>(pl->rows < pl->block_rows ? pl->rows : pl->block_rows);
   // Every sequence has the same q-block count here, so decode_work can map
   // workgroups to items without a list; the heaviest-first order only pays
-  // when the grid runs in more than one round (the decode kernel: one
-  // workgroup per CU; the fp32 kernel: two).  (d1: the 4.8 us plan launch
-  // was 7 % of the step.)
+  // when the grid runs in more than one round (the decode kernels, and any at
+  // head_dim 256: one workgroup per CU; the others two).  (16 x 8192 keys of 8
+  // heads, D64: the 4.8 us plan launch was 7 % of the call.)
   pl->plan = p->layout != FA2_LAYOUT_DENSE;
   pl->dev_splits = false;
   const int64_t resident = pl->dec || pl->decf32 || pl->dim > 128 ? 1 : 2;  // workgroups per CU
@@ -639,8 +639,9 @@ int make_plan_packed(const fa2_params* p, Plan* pl, bool query_device) {
   // Automatic splits: the balanced walk; 16-bit units of up to kDwRows rows
   // then run the wave-streaming kernel.  The ring kernel keeps forced split
   // counts, wait bounds and larger units: at 32 rows two 16-row blocks per wave
-  // were slower (64 sequences of 512-8192 keys, Hq32/Hkv8 D128, 8 drafts: 207 us
-  // ring, 212-226 waves), at 4 rows the waves are faster (207 -> 189).
+  // were slower on a full batch (64 sequences of 512-8192 keys, Hq32/Hkv8 D128,
+  // 8 drafts: 207 us ring, 212-226 waves; smaller batches were not measured), at
+  // 4 rows the waves are faster (207 -> 189).
   const bool wave = pl->dec && pl->rows <= kDwRows && p->decode_spin_cap == 0;
   if ((pl->decf32 || wave) && p->num_splits == 0 && p->batch <= 64 * kWalkMaxPer) {
     const int64_t wgs = cus * (pl->dec4 ? 2 : 1);

@@ -95,15 +95,15 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
   DecPiece p;
   DecSegment sg{};
   if (walk) {
-    if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
+    if (wave == 0) walk_locate<MODE>(a, seg_k, &seg_sh);
     __syncthreads();
     sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
     sg.us = __builtin_amdgcn_readfirstlane(seg_sh.us);
     sg.s0 = __builtin_amdgcn_readfirstlane(seg_sh.s0);
     sg.s1 = __builtin_amdgcn_readfirstlane(seg_sh.s1);
     sg.C = __builtin_amdgcn_readfirstlane(seg_sh.C);
-    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, sg.j, sg.us, p)) return;
-  } else if (!split_piece<MODE, kBN>(a, p)) {
+    if (!walk_piece<MODE>(a, sg, stream, seg_k, sg.j, sg.us, p)) return;
+  } else if (!split_piece<MODE>(a, p)) {
     return;
   }
 
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * NW, kDecF32Waves / 4) void fa2_decode_f32_kern
     if (walk) {
       int j = w.b;
       walk_next_unit(a, sg, j, stream);
-      has_next = walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, p.us + p.W, next);
+      has_next = walk_piece<MODE>(a, sg, stream, seg_k, j, p.us + p.W, next);
     }
     int last[NB];  // last visible key of this lane's row
 #pragma unroll

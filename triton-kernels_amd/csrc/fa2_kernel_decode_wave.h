@@ -28,10 +28,11 @@
 // Measured on MI355X, us per call, against the producer / consumer ring of
 // fa2_kernel_decode.h with a plan kernel or splits: 64 sequences of 512-8192
 // keys Hq32/Hkv8 D128 208 -> 189 (6.15 TB/s; a plain read reaches 6.9), 16 x
-// 8200 keys, 8 heads of D64, 8 drafts 69 -> 58, one sequence of 8000 keys
-// 41 -> 21, 4 x 1023 dense 17.5 -> 12.5.  What is left is uneven service:
-// equal shares end 119 to 184 us into the first of these calls, by kv head
-// (the channels its rows fall on) and by XCD.
+// 8200 keys, 8 heads of D64, 8 drafts 69 -> 59, one sequence of 8000 keys
+// 41 -> 21, 4 x 1023 dense 17.5 -> 12.7, 4 x 500-1500 keys Hkv8 D64 15.8 -> 10.3.
+// Keys are read once (1.00 of their bytes from HBM); what is left is uneven
+// service: equal shares end 121 to 186 us into the first of these calls, by kv
+// head (the channels its rows fall on) and by XCD.
 #pragma once
 
 #include "fa2_decode_walk.h"
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(kDwThreads, 1) void fa2_decode_wave_kernel(KArgs a)
   const int stream = static_cast<int>(blockIdx.x) % a.walk_streams;
   const int seg_k = static_cast<int>(blockIdx.x) / a.walk_streams;
 
-  if (wave == 0) walk_locate<MODE, kBN>(a, seg_k, &seg_sh);
+  if (wave == 0) walk_locate<MODE>(a, seg_k, &seg_sh);
   __syncthreads();
   DecSegment sg;
   sg.j = __builtin_amdgcn_readfirstlane(seg_sh.j);
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(kDwThreads, 1) void fa2_decode_wave_kernel(KArgs a)
     }
   };
   auto first_window = [&](Window& v, int j, int us) -> bool {
-    if (!walk_piece<MODE, kBN>(a, sg, stream, seg_k, j, us, v.p)) return false;
+    if (!walk_piece<MODE>(a, sg, stream, seg_k, j, us, v.p)) return false;
     v.kend = min((v.p.t0 + v.p.T) * kBN, v.p.w.Lk);
     window_at(v, v.p.t0 * kBN);
     return true;
