@@ -135,7 +135,7 @@ def cpu_baseline(w: W.Workload, budget_s: float = 20.0):
 def cpu_threads() -> int:
     """Threads for the CPU baseline: every core of the affinity mask, capped by
     the host's CPU share for this job when the environment states one
-    (OMP_NUM_THREADS; the GPU boxes give one GPU's job 16 cores)."""
+    (OMP_NUM_THREADS)."""
     n = len(os.sched_getaffinity(0))
     share = os.environ.get("OMP_NUM_THREADS", "")
     if share.isdigit() and int(share) > 0:

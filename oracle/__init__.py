@@ -3,7 +3,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Only ``tests/``, ``__graft_entry__.smoke()`` and
 the ``cpu_baseline`` leg of ``bench.py`` import this package, and only as the
-checker.  The product path (``triton-kernels_amd/kernels``) never imports it.
+oracle.  The product path (``triton-kernels_amd/kernels``) never imports it.
 
 Two restatements live here:
 

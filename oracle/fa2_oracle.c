@@ -2,7 +2,7 @@
  * fa2_oracle.c - CPU restatement of harsh-vsingh/triton-kernels
  * `flash_attention_v2` (kernels/attention.py:430-927).
  *
- * TEST INFRASTRUCTURE ONLY.  This file is the checker the parity tests,
+ * TEST INFRASTRUCTURE ONLY.  This file is the oracle the parity tests,
  * `__graft_entry__.smoke()` and bench.py's CPU-baseline leg compare the HIP
  * kernels against.  Nothing in the product path loads it.
  *

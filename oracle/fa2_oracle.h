@@ -5,7 +5,7 @@
  * (kernels/speculative_decode.py:22-365).
  *
  * TEST INFRASTRUCTURE ONLY: used by tests/, __graft_entry__.smoke() and the
- * CPU-baseline leg of bench.py as the checker; never by the product path.
+ * CPU-baseline leg of bench.py as the oracle; never by the product path.
  *
  * Inputs are fp32 host arrays holding values already representable in the
  * tensor dtype under test (an exact upcast of fp16/bf16 data).  Strides and

@@ -1,7 +1,7 @@
 """CPU restatement of the reference's paged-cache construction, and of
 appending rows to such a cache.
 
-TEST INFRASTRUCTURE ONLY (imported by tests/ as the checker of
+TEST INFRASTRUCTURE ONLY (imported by tests/ as the oracle of
 ``kernels.paged_cache``; never by the product path).
 
 * :func:`allocate_paged_cache` follows tests/test_attention.py:101-134 line
